@@ -112,6 +112,10 @@ int nlg_kernel_abi(const char *name, uint32_t *nbuf, uint32_t *npush);
  * constants imply before anything is launched (status NLG_ERR, nothing run, if
  * a buffer is short); data-dependent indices (POS, TOK, TABLE) are bounds-
  * checked on the device (out-of-range reads give 0, writes are dropped).
+ * decode-attn and decode-attn-b of many positions split them over workgroups,
+ * whose partial results meet in a scratch of the library kept per stream (a
+ * few MB, grown on the first such call); a call being captured into a graph
+ * uses none, so such a graph may run beside other calls.
  * Replaces get_kernel (vkserver.c:247-272) plus one vkCmdDispatch
  * (vkserver.c:312-322, vkrun.c:117-123). */
 int nlg_dispatch(const char *name, const nlg_buffer *bufs, uint32_t nbuf,

@@ -2,11 +2,12 @@
 //
 //   decode-attn / decode-attn-b (kernels.el:315-390): single-query causal GQA
 //     over cached K/V.  The reference spends one invocation per output
-//     element and recomputes every q.k product hd times; here a workgroup
-//     owns one (sequence, head): each wave takes every 4th position, its 64
-//     lanes split the head dimension (coalesced 512-byte K/V rows at hd=128),
-//     the q.k product is one DPP reduction, and the four waves' running
-//     (z, ctx) are merged through LDS.
+//     element and recomputes every q.k product hd times; here the positions
+//     are split over workgroups that each serve the query heads of one kv head
+//     (k_decode_split).  Forms that is not made for: a workgroup owns one
+//     (sequence, head), each wave takes every 4th position, its 64 lanes split
+//     the head dimension, the q.k product is one DPP reduction, and the four
+//     waves' running (z, ctx) are merged through LDS (k_decode_attn).
 //   attn-causal-gqa (kernels.el:934-990): 32-query tiles on the f32 matrix
 //     cores; one wave per (head, query) for the forms those do not take.
 //   attn-scores / attn-context (kernels.el:205-235): per element, serial in
@@ -14,6 +15,8 @@
 // Every access is bounds-checked (reads past a buffer give 0, writes are
 // dropped) because POS comes from device memory.
 #include <math.h>
+
+#include <mutex>
 
 #include "nlg_internal.h"
 
@@ -119,6 +122,264 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecArgs a) {
   }
 }
 
+
+// decode-attn(-b) with the positions split: a workgroup takes G query heads of
+// one kv head of one sequence, so a K or V row is read once for them, and its
+// eight waves walk blocks of DS_NI x PPI positions (float4 pieces, L lanes a
+// row, PPI = 64 / L rows an instruction) dealt round-robin over all waves of
+// all `nsplit` workgroups of the unit.  One pass: each block moves the wave's
+// running maximum, sum and context (scores in base 2), the next block's rows
+// already on their way.  With nsplit > 1 the workgroup leaves its partial
+// context and (maximum, sum) for k_decode_merge; with 1 it writes C.
+// Bound by the K/V stream and, below a few MB, by the launches and the chain
+// position -> rows -> partials: 4 sequences of 2,048 positions, 20 heads over 5
+// of 128 (42 MB) 926 -> 22.4 us; one of 701 positions 240 -> 11.6; one of 8,001,
+// 32 heads over 8 (66 MB) 3,680 -> 29.0 (2.3 TB/s); one of 32 9.5 -> 6.9.  k_decode_attn,
+// two passes of one position a wave at a time, stays for buffers that hold no
+// whole float4 rows.
+#define DS_WAVES 8
+#define DS_NI 8
+#define DS_MAX_SPLIT 64  // a merge workgroup's first wave holds one partial a lane
+struct SplitArgs {
+  DecArgs d;
+  uint32_t nsplit, hgroups;  // workgroups per (sequence, kv head, head group); head groups per kv head
+  float *pctx, *pmz;         // [B][heads][nsplit][hd], [B][heads][nsplit][2]
+};
+
+// Sum over aligned groups of L lanes (16, 32 or 64), in every lane.
+template <int L>
+__device__ __forceinline__ float lanes_sum(float v) {
+  v = v + __int_as_float(nlg_dpp<0xB1>(__float_as_int(v)));   // quad_perm [1,0,3,2]
+  v = v + __int_as_float(nlg_dpp<0x4E>(__float_as_int(v)));   // quad_perm [2,3,0,1]
+  v = v + __int_as_float(nlg_dpp<0x141>(__float_as_int(v)));  // row_half_mirror
+  v = v + __int_as_float(nlg_dpp<0x140>(__float_as_int(v)));  // row_mirror
+  if (L >= 32) v = v + __shfl_xor(v, 16);
+  if (L >= 64) v = v + __shfl_xor(v, 32);
+  return v;
+}
+
+template <int L, int G, bool SPLIT>
+__global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
+  constexpr int PPI = 64 / L, PB = DS_NI * PPI;
+  const DecArgs &a = sa.d;
+  __shared__ __align__(16) float s_ctx[DS_WAVES][G][4 * L];
+  __shared__ float s_m[DS_WAVES][G], s_z[DS_WAVES][G];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, sub = lane / L, dl = lane % L;
+  const uint32_t split = SPLIT ? blockIdx.x % sa.nsplit : 0u, unit = SPLIT ? blockIdx.x / sa.nsplit : blockIdx.x;
+  const uint32_t hg = unit % sa.hgroups, kvh = unit / sa.hgroups % a.kvheads, bb = unit / sa.hgroups / a.kvheads;
+  const uint32_t h0 = kvh * a.grp + hg * G, nh = a.grp - hg * G < (uint32_t)G ? a.grp - hg * G : (uint32_t)G;
+  const uint32_t pos = nlg_f2u(ald(a.pos, 0)), len = pos + 1u;
+  const uint64_t base0 = (uint64_t)bb * a.maxseq * a.kvdim;
+  // rows past the caches score 0 with a zero V row: counted at the end
+  const uint64_t rows = base0 < a.ck.n ? (a.ck.n - base0) / a.kvdim : 0;
+  const uint32_t jl = len < rows ? len : (uint32_t)rows;
+  const bool on = 4u * dl < a.hd;
+  const float coef = NLG_LOG2E / sqrtf((float)a.hd);
+  const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float4 q[G], cx[G];
+  float m[G], z[G];
+#pragma unroll
+  for (int h = 0; h < G; h++) {
+    const uint32_t hh = (uint32_t)h < nh ? h0 + h : h0;
+    q[h] = *(const float4 *)(a.q.p + (size_t)bb * a.dim + (size_t)hh * a.hd + (on ? 4 * dl : 0));
+    if (!on) q[h] = zero4;
+    cx[h] = zero4;
+    m[h] = NEG_BIG * NLG_LOG2E;
+    z[h] = 0.0f;
+  }
+  const size_t rb = base0 + kvh * a.hd + (on ? 4 * dl : 0);
+  const float *kp = a.ck.p + rb, *vp = a.cv.p + rb;
+  const uint32_t stride = DS_WAVES * sa.nsplit * PB;
+  uint32_t j0 = (w * sa.nsplit + split) * PB;
+  float4 kn[DS_NI], vn[DS_NI];
+  // rows past the last position fetch the last one again (one cached row)
+  auto load = [&](uint32_t j) {
+#pragma unroll
+    for (int i = 0; i < DS_NI; i++) {
+      const uint32_t r = j + i * PPI + sub, rc = r < jl ? r : jl - 1;
+      kn[i] = *(const float4 *)(kp + (size_t)rc * a.kvdim);
+    }
+#pragma unroll
+    for (int i = 0; i < DS_NI; i++) {
+      const uint32_t r = j + i * PPI + sub, rc = r < jl ? r : jl - 1;
+      vn[i] = *(const float4 *)(vp + (size_t)rc * a.kvdim);
+    }
+  };
+  if (j0 < jl) load(j0);
+  for (; j0 < jl; j0 += stride) {
+    float4 k[DS_NI], v[DS_NI];
+#pragma unroll
+    for (int i = 0; i < DS_NI; i++) {
+      const bool ok = j0 + i * PPI + sub < jl;  // a row not attended may hold anything: its V counts as zeros
+      k[i] = kn[i];
+      v[i] = make_float4(ok ? vn[i].x : 0.0f, ok ? vn[i].y : 0.0f, ok ? vn[i].z : 0.0f, ok ? vn[i].w : 0.0f);
+    }
+    const uint32_t nx = jl - j0 > stride ? j0 + stride : jl - 1;
+    load(nx);
+    float s[DS_NI][G];
+#pragma unroll
+    for (int i = 0; i < DS_NI; i++)
+#pragma unroll
+      for (int h = 0; h < G; h++) {
+        float d = q[h].x * k[i].x;
+        d = fmaf(q[h].y, k[i].y, d);
+        d = fmaf(q[h].z, k[i].z, d);
+        d = fmaf(q[h].w, k[i].w, d);
+        if (!on) d = 0.0f;
+        d = lanes_sum<L>(d);
+        s[i][h] = j0 + i * PPI + sub < jl ? d * coef : -INFINITY;
+      }
+#pragma unroll
+    for (int h = 0; h < G; h++) {
+      float bm = m[h];
+#pragma unroll
+      for (int i = 0; i < DS_NI; i++) bm = s[i][h] > bm ? s[i][h] : bm;  // NaN never becomes the maximum
+      const float al = nlg_exp2(m[h] - bm);
+      m[h] = bm;
+      z[h] *= al;
+      cx[h].x *= al; cx[h].y *= al; cx[h].z *= al; cx[h].w *= al;
+#pragma unroll
+      for (int i = 0; i < DS_NI; i++) {
+        const float e = nlg_exp2(s[i][h] - bm);
+        z[h] += e;
+        cx[h].x = fmaf(e, v[i].x, cx[h].x);
+        cx[h].y = fmaf(e, v[i].y, cx[h].y);
+        cx[h].z = fmaf(e, v[i].z, cx[h].z);
+        cx[h].w = fmaf(e, v[i].w, cx[h].w);
+      }
+    }
+  }
+  // the wave's row slots meet, then the waves
+#pragma unroll
+  for (int h = 0; h < G; h++) {
+#pragma unroll
+    for (int off = L; off < 64; off <<= 1) {
+      const float om = __shfl_xor(m[h], off), mm = om > m[h] ? om : m[h];
+      const float al = nlg_exp2(m[h] - mm), ol = nlg_exp2(om - mm);
+      z[h] = fmaf(z[h], al, __shfl_xor(z[h], off) * ol);
+      cx[h].x = fmaf(cx[h].x, al, __shfl_xor(cx[h].x, off) * ol);
+      cx[h].y = fmaf(cx[h].y, al, __shfl_xor(cx[h].y, off) * ol);
+      cx[h].z = fmaf(cx[h].z, al, __shfl_xor(cx[h].z, off) * ol);
+      cx[h].w = fmaf(cx[h].w, al, __shfl_xor(cx[h].w, off) * ol);
+      m[h] = mm;
+    }
+    if (sub == 0) *(float4 *)&s_ctx[w][h][4 * dl] = cx[h];
+    if (lane == 0) {
+      s_m[w][h] = m[h];
+      s_z[w][h] = z[h];
+    }
+  }
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < nh * a.hd; e += 64 * DS_WAVES) {
+    const uint32_t h = e / a.hd, d = e % a.hd;
+    float mm = s_m[0][h];
+#pragma unroll
+    for (int k = 1; k < DS_WAVES; k++) mm = s_m[k][h] > mm ? s_m[k][h] : mm;
+    const uint32_t out = split == 0 ? len - jl : 0u;  // positions past the caches: score 0, zero V
+    if (out && 0.0f > mm) mm = 0.0f;
+    float zz = out ? (float)out * nlg_exp2(0.0f - mm) : 0.0f, c = 0.0f;
+#pragma unroll
+    for (int k = 0; k < DS_WAVES; k++) {
+      const float sc = nlg_exp2(s_m[k][h] - mm);
+      zz = fmaf(s_z[k][h], sc, zz);
+      c = fmaf(s_ctx[k][h][d], sc, c);
+    }
+    const size_t at = (size_t)bb * a.heads + h0 + h;
+    if (SPLIT) {
+      sa.pctx[(at * sa.nsplit + split) * a.hd + d] = c;
+      if (d == 0) {
+        sa.pmz[(at * sa.nsplit + split) * 2] = mm;
+        sa.pmz[(at * sa.nsplit + split) * 2 + 1] = zz;
+      }
+    } else {
+      const size_t idx = at * a.hd + d;
+      if (idx < a.domain && idx < a.nc) a.c[idx] = c / zz;
+    }
+  }
+}
+
+// The workgroups' partials of one (sequence, head), merged and normalised.
+__global__ __launch_bounds__(256) void k_decode_merge(SplitArgs sa) {
+  const DecArgs &a = sa.d;
+  __shared__ float s_w[DS_MAX_SPLIT], s_z;
+  const size_t at = blockIdx.x;
+  if (threadIdx.x < 64) {
+    const uint32_t t = threadIdx.x;
+    const float *mz = sa.pmz + at * sa.nsplit * 2;
+    const float m = t < sa.nsplit ? mz[2 * t] : NEG_BIG * NLG_LOG2E, z = t < sa.nsplit ? mz[2 * t + 1] : 0.0f;
+    const float sc = nlg_exp2(m - nlg_wave_max_f32(m));
+    s_w[t] = sc;
+    const float zz = nlg_wave_sum_f32(z * sc);
+    if (t == 0) s_z = zz;
+  }
+  __syncthreads();
+  const float *pc = sa.pctx + at * sa.nsplit * a.hd;
+  for (uint32_t d = threadIdx.x; d < a.hd; d += 256) {
+    float c = 0.0f;
+#pragma unroll 8
+    for (uint32_t k = 0; k < sa.nsplit; k++) c = fmaf(pc[(size_t)k * a.hd + d], s_w[k], c);
+    const size_t idx = at * a.hd + d;
+    if (idx < a.domain && idx < a.nc) a.c[idx] = c / s_z;
+  }
+}
+
+template <int L, bool SPLIT>
+static void decode_split_go(const SplitArgs &sa, uint32_t g, hipStream_t st) {
+  const dim3 grid(sa.d.B * sa.d.kvheads * sa.hgroups * sa.nsplit), blk(64 * DS_WAVES);
+  if (g == 4) hipLaunchKernelGGL((k_decode_split<L, 4, SPLIT>), grid, blk, 0, st, sa);
+  else if (g == 2) hipLaunchKernelGGL((k_decode_split<L, 2, SPLIT>), grid, blk, 0, st, sa);
+  else hipLaunchKernelGGL((k_decode_split<L, 1, SPLIT>), grid, blk, 0, st, sa);
+}
+template <bool SPLIT>
+static void decode_split_hd(const SplitArgs &sa, uint32_t g, hipStream_t st) {
+  if (sa.d.hd <= 64) decode_split_go<16, SPLIT>(sa, g, st);
+  else if (sa.d.hd <= 128) decode_split_go<32, SPLIT>(sa, g, st);
+  else decode_split_go<64, SPLIT>(sa, g, st);
+}
+
+// Whether k_decode_split takes this call (whole float4 rows, unchecked: the
+// caches hold whole rows, as many of K as of V; q and every head's output
+// columns exist), and its launches.  The partials live in a scratch of the
+// stream; the mutex keeps two threads' launch pairs on one stream apart.  A
+// call that is being captured, or whose scratch cannot be had, runs with one
+// workgroup per unit, in one launch and without scratch: a graph may be
+// replayed beside other calls.
+static bool decode_split(const DecArgs &a, hipStream_t st) {
+  const uintptr_t at = (uintptr_t)a.q.p | (uintptr_t)a.ck.p | (uintptr_t)a.cv.p;
+  if (a.hd % 4 || a.hd > 256 || a.dim != a.heads * a.hd || a.heads % a.kvheads || !a.q.p || !a.ck.p || !a.cv.p ||
+      (at & 15) || a.ck.n != a.cv.n || a.ck.n % a.kvdim || a.q.n < (uint64_t)a.B * a.dim ||
+      (uint64_t)a.B * a.dim >= (1u << 31) || (uint64_t)a.B * a.maxseq * a.kvdim > 0xffffffffull)
+    return false;
+  SplitArgs sa{};
+  sa.d = a;
+  // four heads a workgroup, unless that leaves half of its registers idle
+  const uint32_t g = a.grp >= 3 ? 4u : a.grp;
+  sa.hgroups = (a.grp + g - 1) / g;
+  sa.nsplit = 1;
+  // two workgroups per CU, none with less than a block for each wave
+  const uint64_t units = (uint64_t)a.B * a.kvheads * sa.hgroups, rows = a.maxseq ? a.maxseq : a.ck.n / a.kvdim;
+  const uint32_t pb = DS_NI * (a.hd <= 64 ? 4u : a.hd <= 128 ? 2u : 1u);
+  uint64_t want = 2ull * nlg_num_cu() / units, most = (rows + DS_WAVES * pb - 1) / (DS_WAVES * pb);
+  if (want > DS_MAX_SPLIT) want = DS_MAX_SPLIT;
+  if (want > most) want = most;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (want > 1 && hipStreamIsCapturing(st, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone) {
+    const size_t n = (size_t)a.B * a.heads * want;
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lk(mu);
+    if (float *ws = (float *)nlg_scratch_try((n * a.hd + 2 * n) * 4, st, 3)) {
+      sa.nsplit = (uint32_t)want;
+      sa.pctx = ws;
+      sa.pmz = ws + n * a.hd;
+      decode_split_hd<true>(sa, g, st);
+      hipLaunchKernelGGL(k_decode_merge, dim3(a.B * a.heads), dim3(256), 0, st, sa);
+      return true;
+    }
+  }
+  decode_split_hd<false>(sa, g, st);
+  return true;
+}
+
 static int decode_attn_common(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipStream_t st,
                               bool batched) {
   DecArgs a;
@@ -145,6 +406,10 @@ static int decode_attn_common(const nlg_buffer *b, const uint32_t *p, uint32_t g
   a.c = (float *)b[4].ptr;
   a.nc = b[4].nfloats;
   const uint32_t seqs = (uint32_t)((dom + a.dim - 1) / a.dim);
+  if (decode_split(a, st)) {
+    NLG_LAUNCHED(k);
+    return NLG_OK;
+  }
   dim3 g(seqs * a.hslots), blk(256);
   if (a.hd <= 64) hipLaunchKernelGGL(k_decode_attn<1>, g, blk, 0, st, a);
   else if (a.hd <= 128) hipLaunchKernelGGL(k_decode_attn<2>, g, blk, 0, st, a);

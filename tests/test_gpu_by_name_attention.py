@@ -2,7 +2,10 @@
 32, 64, 80, 96, 128) against the CPU restatement, at the sizes where it can go
 wrong: the edges of its 32-query tiles and 32-key blocks, one to four key
 blocks per wave, every instantiated head dim, partial grids, a V of infinities
-and NaNs after a query, and buffers that take the general kernel instead."""
+and NaNs after a query, and buffers that take the general kernel instead.
+decode-attn(-b) on its split form likewise: every lanes-per-row form, one and
+many workgroups per head (a call under capture takes one), positions at the
+edges of its blocks and past the cache, NaN in every row not attended."""
 import numpy as np
 import pytest
 
@@ -113,3 +116,105 @@ def test_prompt_attention_f32_general_form(form):
     want = out.copy()
     orc.dispatch("attn-causal-gqa", [q.copy(), k.copy(), short, want], push, groups)
     assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+def decode_inputs(batch, heads, kvh, hd, maxseq, seed=0):
+    rng = np.random.default_rng(batch * 31 + heads * 7 + hd + maxseq + seed)
+    q = (rng.standard_normal(batch * heads * hd) * 1.5).astype(f32)
+    n = batch * maxseq * kvh * hd
+    return q, rng.standard_normal(n).astype(f32), rng.standard_normal(n).astype(f32)
+
+
+def decode_both(q, k, v, pos, push, groups=None, fill=0.0, stale=np.nan, graph=False):
+    """The split decode attention and the oracle; rows past `pos` of every
+    sequence hold `stale` on the device (nobody attends them)."""
+    batch, dim, heads, kvh, maxseq = push
+    kvd = kvh * (dim // heads)
+    kd, vd = k.copy(), v.copy()
+    for x in (kd, vd):
+        x.reshape(batch, maxseq, kvd)[:, pos + 1:] = stale
+    out = np.full(batch * dim, fill, f32)
+    devs = [nlgpu.to_device(b) for b in (q, kd, vd, np.array([pos], f32), out)]
+    groups = (batch * dim + 63) // 64 if groups is None else groups
+    if graph:
+        s = nlgpu.lib().nlg_stream_create()
+        nlgpu.graph_begin(s)
+        nlgpu.dispatch("decode-attn-b", devs, push, groups, stream=s)
+        g = nlgpu.graph_end(s)
+        for _ in range(3):
+            devs[-1].upload(out)
+            nlgpu.graph_launch(g, s)
+            nlgpu.sync(s)
+        nlgpu.graph_destroy(g)
+        nlgpu.lib().nlg_stream_destroy(s)
+    else:
+        nlgpu.dispatch("decode-attn-b", devs, push, groups)
+    got = devs[-1].download(f32, out.size)
+    want = out.copy()
+    orc.dispatch("decode-attn-b", [q.copy(), k.copy(), v.copy(), np.array([pos], f32), want], push, groups)
+    return got, want
+
+
+# sums of up to 1,500 terms, the error of a random order about sqrt(1500) x
+# 2^-24 = 2e-6 of the output: the 1e-5 bar the by-name cases state
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("batch,heads,kvh,hd,maxseq,pos", [
+    (1, 4, 1, 128, 40, 0), (2, 4, 2, 128, 300, 15), (1, 20, 5, 128, 1500, 1499), (3, 6, 2, 64, 700, 511),
+    (2, 8, 8, 80, 260, 129), (1, 14, 2, 96, 600, 513), (2, 4, 2, 256, 200, 64), (40, 16, 16, 32, 33, 20),
+    (1, 5, 5, 20, 77, 76)])
+def test_decode_attention_f32(batch, heads, kvh, hd, maxseq, pos, graph):
+    print(f"[gpu] decode-attn-b batch={batch} heads={heads}/{kvh} hd={hd} pos={pos}/{maxseq} graph={graph}", flush=True)
+    q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq)
+    got, want = decode_both(q, k, v, pos, [batch, heads * hd, heads, kvh, maxseq], graph=graph)
+    assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("pos", [299, 300, 1000])
+def test_decode_attention_f32_past_the_cache(pos):
+    """Positions past the last sequence's rows read as zeros: score 0, no V."""
+    batch, heads, kvh, hd, maxseq = 1, 4, 2, 64, 300
+    q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq)
+    got, want = decode_both(q, k, v, pos, [batch, heads * hd, heads, kvh, maxseq])
+    assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+def test_decode_attention_f32_partial_grid_and_single():
+    batch, heads, kvh, hd, maxseq, pos = 3, 4, 2, 64, 130, 100
+    q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq)
+    got, want = decode_both(q, k, v, pos, [batch, heads * hd, heads, kvh, maxseq], groups=5, fill=-7.0)
+    assert np.array_equal(got[320:], want[320:]) and np.all(want[320:] == -7.0)
+    assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
+    one = maxseq * kvh * hd
+    out = np.zeros(heads * hd, f32)
+    bufs = [q[:heads * hd], k[:one], v[:one], np.array([pos], f32), out]
+    devs = [nlgpu.to_device(b) for b in bufs]
+    nlgpu.dispatch("decode-attn", devs, [heads * hd, heads, kvh], 4)
+    want = out.copy()
+    orc.dispatch("decode-attn", [b.copy() for b in bufs[:4]] + [want], [heads * hd, heads, kvh], 4)
+    assert np.max(np.abs(devs[-1].download(f32, out.size) - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+def test_decode_attention_f32_infinities():
+    """An attended V of infinities and an attended K whose score is NaN."""
+    batch, heads, kvh, hd, maxseq, pos = 1, 4, 2, 64, 200, 150
+    for bad in ("v", "k"):
+        q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq)
+        x = (v if bad == "v" else k).reshape(maxseq, kvh, hd)
+        x[40, 0, :] = np.inf if bad == "v" else np.nan
+        got, want = decode_both(q, k, v, pos, [batch, heads * hd, heads, kvh, maxseq])
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        fine = np.isfinite(want)
+        assert fine.any() and not fine.all()
+        assert np.max(np.abs(got[fine] - want[fine])) <= 1e-5 * np.max(np.abs(want[fine]))
+
+
+def test_decode_attention_f32_general_form():
+    """K shorter than V by part of a row: the general kernel (zeros past it)."""
+    batch, heads, kvh, hd, maxseq, pos = 1, 4, 2, 64, 90, 89
+    q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq)
+    push, out = [batch, heads * hd, heads, kvh, maxseq], np.zeros(heads * hd, f32)
+    devs = [nlgpu.to_device(b) for b in (q, k, v, np.array([pos], f32), out)]
+    nlgpu.dispatch("decode-attn-b", [devs[0], (devs[1], k.size - 70)] + devs[2:], push, 4)
+    want = out.copy()
+    orc.dispatch("decode-attn-b", [q.copy(), k[:k.size - 70].copy(), v.copy(), np.array([pos], f32), want], push, 4)
+    assert np.max(np.abs(devs[-1].download(f32, out.size) - want)) <= 1e-5 * np.max(np.abs(want))
