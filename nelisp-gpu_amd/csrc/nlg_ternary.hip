@@ -19,6 +19,8 @@
 // 16 columns, done once per wave and reused for every row).  The int32 sum
 // is therefore 64x the exact accumulator and `>> 6` recovers it exactly;
 // the fp32 epilogue is bitlinear-dp4a-1f's, evaluated without contraction.
+#include <type_traits>
+
 #include "nlg_quant.h"
 
 // ------------------------------------------------------------ quantisation
@@ -677,39 +679,252 @@ int L_dp4a_dot(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipStrea
 // ------------------------------------------------------ f32-activation linears
 
 // ternary-rows (kernels.el:700-746): f32 activations, 2-bit weights, one
-// scale per 128-column block.  One wave per output; lane-partial sums are
-// scaled per word by the word's block beta (reassociated: tolerance parity).
-__global__ __launch_bounds__(256) void k_ternary_rows(const float *x, const uint32_t *wp,
-                                                      const float *bias, const float *beta, float *y,
-                                                      uint32_t n_out, uint32_t out, uint32_t cols,
-                                                      uint32_t nblk, uint32_t wng) {
+// scale per 128-column block (reassociated: tolerance parity).
+struct TRowsArgs {
+  const float *x;
+  const uint32_t *wp;
+  const float *bias, *beta;
+  float *y;
+  uint64_t n;  // outputs written: row-major index below n
+  uint32_t seq, out, cols, nblk, wng;
+  uint32_t nw;  // words of a row that count: b*8 + w < wng for b < nblk only
+};
+
+// Few tokens: a wave owns R rows for T tokens, lane l word l (+ 64 k) of each
+// row, whose fields are decoded once for the T tokens while the 16 columns of
+// x sit in registers.  Per lane and word the products are added in field
+// order, then scaled, then the lanes' sums meet: the sums of the former kernel
+// (one output a wave, x gathered and the weights decoded per token), bit for
+// bit.  6,912 x 2,560: 1 token 6.9 us, 2 tokens 7.4.
+// XV: x rows are 16-byte aligned and a multiple of 4 long.
+template <int R, int T, bool XV>
+__global__ __launch_bounds__(256) void k_ternary_rows(TRowsArgs a) {
   const int lane = threadIdx.x & 63;
-  const uint64_t wave = (uint64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (wave >= n_out) return;
-  const uint32_t idx = (uint32_t)wave, s = idx / out, o = idx % out;
-  const float *xr = x + (size_t)s * cols;
-  const uint32_t *wr = wp + (size_t)o * wng;
-  // the reference visits words wi = b*8 + w < wng for b < nblk only
-  const uint32_t nw = wng < 8u * nblk ? wng : 8u * nblk;
-  float acc = 0.0f;
-  for (uint32_t wi = lane; wi < ((nw + 63) & ~63u); wi += 64) {
-    if (wi < nw) {
-      const uint32_t w = wr[wi];
-      float part = 0.0f;
+  const uint32_t nt = (a.out + 4 * R - 1) / (4 * R);
+  const uint32_t o0 = (blockIdx.x % nt * 4 + (threadIdx.x >> 6)) * R, s0 = blockIdx.x / nt * T;
+  if (o0 >= a.out) return;
+  float acc[R][T];
 #pragma unroll
-      for (uint32_t f = 0; f < 16; f++) {
-        const uint32_t i = wi * 16 + f;
-        if (i < cols) {
-          const float sv = (float)((int32_t)(w << (30 - 2 * f)) >> 30);
-          part = __fadd_rn(part, __fmul_rn(sv, xr[i]));
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int t = 0; t < T; t++) acc[r][t] = 0.0f;
+  for (uint32_t wb = 0; wb < a.nw; wb += 64) {
+    const uint32_t wi = wb + lane < a.nw ? wb + lane : a.nw - 1, c0 = wi * 16;
+    uint32_t w[R];
+    float be[R], x[T][16];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const size_t o = o0 + r < a.out ? o0 + r : a.out - 1;
+      w[r] = a.wp[o * a.wng + wi];
+      be[r] = a.beta[o * a.nblk + wi / 8];
+    }
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+      const float *xr = a.x + (size_t)(s0 + t < a.seq ? s0 + t : a.seq - 1) * a.cols;
+      if (XV) {
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+          const uint32_t i = c0 + 4 * f, ic = i < a.cols ? i : a.cols - 4;
+          const float4 v = *(const float4 *)(xr + ic);
+          const bool ok = i < a.cols;
+          x[t][4 * f] = ok ? v.x : 0.0f; x[t][4 * f + 1] = ok ? v.y : 0.0f;
+          x[t][4 * f + 2] = ok ? v.z : 0.0f; x[t][4 * f + 3] = ok ? v.w : 0.0f;
+        }
+      } else {
+#pragma unroll
+        for (int f = 0; f < 16; f++) {
+          const uint32_t i = c0 + f;
+          x[t][f] = i < a.cols ? xr[i] : 0.0f;
         }
       }
-      acc = __fadd_rn(acc, __fmul_rn(beta[(size_t)o * nblk + wi / 8], part));
+    }
+    const bool on = wb + lane < a.nw;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      float part[T];
+#pragma unroll
+      for (int t = 0; t < T; t++) part[t] = 0.0f;
+#pragma unroll
+      for (int f = 0; f < 16; f++) {
+        const float sv = (float)((int32_t)(w[r] << (30 - 2 * f)) >> 30);
+#pragma unroll
+        for (int t = 0; t < T; t++) part[t] = __fadd_rn(part[t], __fmul_rn(sv, x[t][f]));
+      }
+#pragma unroll
+      for (int t = 0; t < T; t++)
+        if (on) acc[r][t] = __fadd_rn(acc[r][t], __fmul_rn(be[r], part[t]));
     }
   }
-  acc = nlg_wave_sum_f32(acc);
-  if (lane == 0) y[idx] = __fadd_rn(bias[o], acc);
+#pragma unroll
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int t = 0; t < T; t++) {
+      const float v = nlg_wave_sum_f32(acc[r][t]);
+      const uint64_t idx = (uint64_t)(s0 + t) * a.out + o0 + r;
+      if (lane == 0 && o0 + r < a.out && s0 + t < a.seq && idx < a.n) a.y[idx] = __fadd_rn(a.bias[o0 + r], v);
+    }
 }
+
+// More tokens: 32 tokens x 32 RB rows a workgroup on v_mfma_f32_32x32x16_bf16
+// (lane 32g + i holds A[i][8g..8g+7] and B[8g..8g+7][i], result r of lane 32g + i
+// is C[(r % 4) + 8 (r / 4) + 4 g][i]), A the activations, B the weights, the NW
+// waves every NW-th 128-column block.
+//  * The weights {-2, -1, 0, 1} are exact in bf16 (byte permutes out of two
+//    four-entry tables).  An activation is split by truncation into three bf16
+//    values of 8 significant bits each, x = hi + mid + lo exactly, so every
+//    product is exact and the sums are f32 as before; hi has its own
+//    accumulator, so the small parts' additions round at their own size (all
+//    in one: error against 64 bits 1.2e-07, apart 6.8e-08, before 1.0e-07).
+//  * Step t of a block contracts word t of each row: lane half g takes fields
+//    8g..8g+7, in the order 0 4 1 5 2 6 3 7 the tables' bytes come out in, and x
+//    is packed alike.  A step's registers are loaded for the wave's next block
+//    as soon as it has used them.
+//  * Per block the sum is scaled by the row's beta and added to the wave's total
+//    in LDS (registers hold no more), where the waves' totals then meet.
+// An infinity's remainders are NaN, so every output that sees one is NaN: such
+// outputs are summed again, one by one, in plain f32.
+// Bound by the vector unit (the split of x, 44 instructions a step, and the
+// decode of the weights, 14 a row block, against 96 matrix-core cycles a row
+// block).  6,912 x 2,560: 64 tokens 1,929 -> 17.1 us (133 TFLOP/s), 16 tokens
+// 10.2, 128 tokens 30; 6,912 x 6,912 at 256 tokens 116 us (211 TFLOP/s).  Four
+// waves with the next block's registers loaded whole took 20.4 us at 64 tokens.
+template <int RB, int NW, bool WVEC>
+__global__ __launch_bounds__(64 * NW) void k_ternary_mfma(TRowsArgs a) {
+  typedef float v16f __attribute__((ext_vector_type(16)));
+  typedef __bf16 v8b __attribute__((ext_vector_type(8)));
+  typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+  __shared__ float s_c[NW][RB][32][33];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, g = lane >> 5, i = lane & 31;
+  const uint32_t nt = (a.out + 32 * RB - 1) / (32 * RB);
+  const uint32_t o0 = blockIdx.x % nt * 32 * RB, s0 = blockIdx.x / nt * 32;
+  const uint32_t keff = a.cols < a.nw * 16 ? a.cols : a.nw * 16, nb = (a.nw + 7) / 8;
+  const float *xr = a.x + (size_t)(s0 + i < a.seq ? s0 + i : a.seq - 1) * a.cols;
+  const uint32_t *wr[RB];
+  const float *br[RB];
+#pragma unroll
+  for (int n = 0; n < RB; n++) {
+    const uint32_t o = o0 + 32 * n + i;
+    wr[n] = a.wp + (size_t)(o < a.out ? o : a.out - 1) * a.wng;
+    br[n] = a.beta + (size_t)(o < a.out ? o : a.out - 1) * a.nblk;
+  }
+  float4 xn[8][2];
+  uint32_t wn[RB][8];
+  auto load_x = [&](uint32_t b, int t) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const uint32_t k = 128 * b + 16 * t + 8 * g + 4 * h;
+      xn[t][h] = *(const float4 *)(xr + (k < keff ? k : keff - 4));
+    }
+  };
+  auto load_w = [&](uint32_t b, int h) {  // words 4h..4h+3 of the block
+#pragma unroll
+    for (int n = 0; n < RB; n++) {
+      if (WVEC) {
+        const uint32_t k = 8 * b + 4 * h;
+        const uint4 v = *(const uint4 *)(wr[n] + (k < a.nw ? k : a.nw - 4));
+        wn[n][4 * h] = v.x; wn[n][4 * h + 1] = v.y; wn[n][4 * h + 2] = v.z; wn[n][4 * h + 3] = v.w;
+      } else {
+#pragma unroll
+        for (int t = 4 * h; t < 4 * h + 4; t++) wn[n][t] = wr[n][8 * b + t < a.nw ? 8 * b + t : a.nw - 1];
+      }
+    }
+  };
+  auto tot = [&](int n, int r) -> float & { return s_c[wv][n][(r % 4) + 8 * (r / 4) + 4 * g][i]; };
+#pragma unroll
+  for (int n = 0; n < RB; n++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) tot(n, r) = 0.0f;
+  if ((uint32_t)wv < nb) {
+    load_w(wv, 0);
+    load_w(wv, 1);
+#pragma unroll
+    for (int t = 0; t < 8; t++) load_x(wv, t);
+  }
+  for (uint32_t b = wv; b < nb; b += NW) {
+    const uint32_t bx = b + NW < nb ? b + NW : b;
+    v16f hi[RB], lo[RB];
+    float be[RB];
+#pragma unroll
+    for (int n = 0; n < RB; n++) {
+#pragma unroll
+      for (int r = 0; r < 16; r++) hi[n][r] = lo[n][r] = 0.0f;
+      be[n] = br[n][b];
+    }
+    auto block = [&](auto full) {  // full: no column of the block lies past the row
+#pragma unroll
+      for (int t = 0; t < 8; t++) {
+        float x[8] = {xn[t][0].x, xn[t][0].y, xn[t][0].z, xn[t][0].w, xn[t][1].x, xn[t][1].y, xn[t][1].z, xn[t][1].w};
+        if (!full.value) {
+#pragma unroll
+          for (int e = 0; e < 8; e++) x[e] = 128 * b + 16 * t + 8 * g + e < keff ? x[e] : 0.0f;
+        }
+        v4u px[3];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          float u = x[e], v = x[e + 4];
+#pragma unroll
+          for (int q = 0; q < 3; q++) {
+            px[q][e] = __builtin_amdgcn_perm(__float_as_uint(v), __float_as_uint(u), 0x07060302u);
+            if (q == 2) break;
+            u = u - __uint_as_float(__float_as_uint(u) & 0xffff0000u);
+            v = v - __uint_as_float(__float_as_uint(v) & 0xffff0000u);
+          }
+        }
+        load_x(bx, t);
+#pragma unroll
+        for (int n = 0; n < RB; n++) {
+          const uint32_t h = wn[n][t] >> (16 * g);
+          v4u pw;
+#pragma unroll
+          for (int q = 0; q < 2; q++) {
+            const uint32_t sel = (q ? (h >> 4 & 0xfffu) | h << 10 : (h & 0xffffu) | h << 14) & 0x03030303u;
+            const uint32_t ph = __builtin_amdgcn_perm(0u, 0xbfc03f00u, sel), pl = __builtin_amdgcn_perm(0u, 0x80008000u, sel);
+            pw[2 * q] = __builtin_amdgcn_perm(ph, pl, 0x05010400u);
+            pw[2 * q + 1] = __builtin_amdgcn_perm(ph, pl, 0x07030602u);
+          }
+          const v8b bw = __builtin_bit_cast(v8b, pw);
+          lo[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, px[2]), bw, lo[n], 0, 0, 0);
+          hi[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, px[0]), bw, hi[n], 0, 0, 0);
+          lo[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8b, px[1]), bw, lo[n], 0, 0, 0);
+        }
+        if (t % 4 == 3) load_w(bx, t / 4);
+      }
+    };
+    if (128 * b + 128 <= keff) block(std::true_type());
+    else block(std::false_type());
+#pragma unroll
+    for (int n = 0; n < RB; n++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) tot(n, r) = fmaf(be[n], hi[n][r] + lo[n][r], tot(n, r));
+  }
+  __syncthreads();
+  for (uint32_t e = threadIdx.x; e < 32 * 32 * RB; e += 64 * NW) {
+    const uint32_t t = e / (32 * RB), n = e / 32 % RB, j = e % 32, s = s0 + t, o = o0 + 32 * n + j;
+    const uint64_t idx = (uint64_t)s * a.out + o;
+    if (s >= a.seq || o >= a.out || idx >= a.n) continue;
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NW; k++) v += s_c[k][n][t][j];
+    if (v != v) {
+      v = 0.0f;
+      for (uint32_t b = 0; b < nb; b++) {
+        float part = 0.0f;
+        for (uint32_t c = 128 * b; c < 128 * b + 128 && c < keff; c++) {
+          const uint32_t w = a.wp[(size_t)o * a.wng + c / 16];
+          part += (float)((int32_t)(w << (30 - 2 * (c % 16))) >> 30) * a.x[(size_t)s * a.cols + c];
+        }
+        v += a.beta[(size_t)o * a.nblk + b] * part;
+      }
+    }
+    a.y[idx] = __fadd_rn(a.bias[o], v);
+  }
+}
+
+// From this many tokens the matrix cores win: 6,912 x 2,560 at 2 / 4 / 8 tokens
+// 8.4 / 8.5 / 8.9 us against 7.3 / 11.2 / 21.2 with four tokens a wave, 2,560 x
+// 6,900 at 64 tokens 26 against 90.  The one loss is a few long rows: 1,000 x
+// 6,912 at 4 / 16 tokens 18.4 / 21.0 against 16.1 / 16.4.
+#define TROWS_MFMA 4
 
 int L_ternary_rows(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipStream_t st) {
   const uint32_t seq = p[0], out = p[1], cols = p[2], nblk = p[3], wng = p[4];
@@ -722,9 +937,37 @@ int L_ternary_rows(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipS
   if (nlg_need(b, 0, xneed, k) || nlg_need(b, 1, (uint64_t)(out - 1) * wng + nw, k) ||
       nlg_need(b, 2, out, k) || nlg_need(b, 3, (uint64_t)out * nblk, k) || nlg_need(b, 4, n, k))
     return NLG_ERR;
-  hipLaunchKernelGGL(k_ternary_rows, dim3(nlg_blocks(n, 4)), dim3(256), 0, st,
-                     (const float *)b[0].ptr, (const uint32_t *)b[1].ptr, (const float *)b[2].ptr,
-                     (const float *)b[3].ptr, (float *)b[4].ptr, (uint32_t)n, out, cols, nblk, wng);
+  TRowsArgs a{(const float *)b[0].ptr, (const uint32_t *)b[1].ptr, (const float *)b[2].ptr, (const float *)b[3].ptr,
+              (float *)b[4].ptr, n, (uint32_t)srows, out, cols, nblk, wng, nw};
+  const bool xv = cols % 4 == 0 && ((uintptr_t)a.x & 15) == 0 && cols;
+  const dim3 blk(256);
+  if (xv && nw && srows >= TROWS_MFMA) {
+    const bool wvec = wng % 4 == 0 && ((uintptr_t)a.wp & 15) == 0;
+    // The smallest tiles that one round of workgroups covers, the largest past
+    // that: 32- / 64-row tiles 10.2 / 13.4 us at 216 / 108 tiles, 25.9 / 17.1 at
+    // 432 / 216; 64- / 128-row tiles 32 / 28 us at 432 / 216, 139 / 106 at 864 / 432.
+    const uint64_t tt = (srows + 31) / 32, cu = nlg_num_cu();
+    const uint32_t rb = tt * ((out + 31) / 32) <= cu ? 1u : tt * ((out + 63) / 64) <= cu ? 2u : 4u;
+    const dim3 g((uint32_t)(tt * ((out + 32 * rb - 1) / (32 * rb))));
+    if (rb == 1 && wvec) hipLaunchKernelGGL((k_ternary_mfma<1, 8, true>), g, dim3(512), 0, st, a);
+    else if (rb == 1) hipLaunchKernelGGL((k_ternary_mfma<1, 8, false>), g, dim3(512), 0, st, a);
+    else if (rb == 2 && wvec) hipLaunchKernelGGL((k_ternary_mfma<2, 8, true>), g, dim3(512), 0, st, a);
+    else if (rb == 2) hipLaunchKernelGGL((k_ternary_mfma<2, 8, false>), g, dim3(512), 0, st, a);
+    else if (wvec) hipLaunchKernelGGL((k_ternary_mfma<4, 4, true>), g, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((k_ternary_mfma<4, 4, false>), g, dim3(256), 0, st, a);
+  } else {
+    const uint32_t t = srows >= 3 ? 4u : (uint32_t)srows;
+    const dim3 g((uint32_t)((srows + t - 1) / t * ((out + 15) / 16)));
+    if (xv) {
+      if (t == 4) hipLaunchKernelGGL((k_ternary_rows<4, 4, true>), g, blk, 0, st, a);
+      else if (t == 2) hipLaunchKernelGGL((k_ternary_rows<4, 2, true>), g, blk, 0, st, a);
+      else hipLaunchKernelGGL((k_ternary_rows<4, 1, true>), g, blk, 0, st, a);
+    } else {
+      if (t == 4) hipLaunchKernelGGL((k_ternary_rows<4, 4, false>), g, blk, 0, st, a);
+      else if (t == 2) hipLaunchKernelGGL((k_ternary_rows<4, 2, false>), g, blk, 0, st, a);
+      else hipLaunchKernelGGL((k_ternary_rows<4, 1, false>), g, blk, 0, st, a);
+    }
+  }
   NLG_LAUNCHED(k);
   return NLG_OK;
 }
