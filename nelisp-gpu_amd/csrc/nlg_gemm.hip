@@ -9,11 +9,12 @@
 //   matmul-tiled                per 16-wide k tile, p0 + (p1 + (... + (p14 +
 //                               p15))) added to acc (the tile sum the
 //                               reference writes out, zero products past K).
-// The chain length bounds the time, not the flops, so the work is spread
-// as wide as it goes: one 256-thread workgroup per 16 x 16 output tile (a
-// 256^3 product is 256 workgroups, one per CU), one output per thread, the
+// In small products the chain length bounds the time, not the flops, so the
+// work is spread as wide as it goes: one 256-thread workgroup per 16 x 16 output
+// tile (a 256^3 product is 256 workgroups, one per CU), one output per thread, the
 // tile's A rows and B columns for 256 values of k staged through LDS with
-// every global load of a chunk issued before the first is used.
+// every global load of a chunk issued before the first is used.  Products of
+// more tiles give a thread several outputs (k_mmt).
 //
 // Partial grids: a dispatch of `groups` workgroups covers only the outputs
 // the reference's invocations gid < 64*groups (matmul-tiled: workgroups
@@ -27,6 +28,14 @@ enum { MM_SERIAL = 0, MM_TILE16 = 1 };
 // which outputs a partial grid covers: by row-major index, by 4x4 block
 // index (matmul-reg), or by 16x16 tile index (matmul-tiled)
 enum { LIM_INDEX = 0, LIM_BLOCK4 = 1, LIM_TILE16 = 2 };
+
+__device__ __forceinline__ bool mm_covered(uint32_t row, uint32_t col, uint32_t N, int lim_mode, uint64_t lim) {
+  uint64_t at;
+  if (lim_mode == LIM_INDEX) at = (uint64_t)row * N + col;
+  else if (lim_mode == LIM_BLOCK4) at = (uint64_t)(row / 4) * ((N + 3) / 4) + col / 4;
+  else at = (uint64_t)(row / 16) * ((N + 15) / 16) + col / 16;
+  return at < lim;
+}
 
 template <int ORDER, bool TRANS_B, bool BIAS>
 __global__ __launch_bounds__(256) void k_mm(const float *__restrict__ A, const float *__restrict__ B,
@@ -81,12 +90,176 @@ __global__ __launch_bounds__(256) void k_mm(const float *__restrict__ A, const f
       }
     }
   }
-  if (row >= M || col >= N) return;
-  uint64_t at;
-  if (lim_mode == LIM_INDEX) at = (uint64_t)row * N + col;
-  else if (lim_mode == LIM_BLOCK4) at = (uint64_t)(row / 4) * ((N + 3) / 4) + col / 4;
-  else at = (uint64_t)(row / 16) * ((N + 15) / 16) + col / 16;
-  if (at < lim) C[(size_t)row * N + col] = acc;
+  if (row < M && col < N && mm_covered(row, col, N, lim_mode, lim)) C[(size_t)row * N + col] = acc;
+}
+
+// The same products and sums with TM x TN outputs a thread, for products large
+// enough to fill the chip that way: a 16 TM x 16 TN tile per workgroup, A and B for
+// 32 values of k staged in LDS (A transposed, so a thread's rows are one read),
+// the next stage's loads in flight, and the LDS reads of four k ahead of the
+// arithmetic.  The multiply and the add round apart, so two vector instructions
+// per product bound it (79 TFLOP/s with every SIMD issuing from several waves: one
+// wave alone issues half as often), and a thread's TM + TN values of a k serve
+// TM x TN products.  1,024^3 134 -> 56 us (38 TFLOP/s), 2,048^3 1,024 -> 349 (49).
+// 8 x 8 outputs a thread leave one wave per SIMD: 560 us at 2,048^3.
+constexpr int MT_KC = 32, MT_KG = 4;  // k per stage; k read ahead
+
+template <int TM, int TN, int ORDER, bool TRANS_B, bool BIAS, bool VEC>
+__global__ __launch_bounds__(256) void k_mmt(const float *__restrict__ A, const float *__restrict__ B,
+                                             const float *__restrict__ bias, float *__restrict__ C, uint32_t M,
+                                             uint32_t N, uint32_t K, int lim_mode, uint64_t lim) {
+  constexpr int TA = 16 * TM, TB = 16 * TN, KC = MT_KC, KG = MT_KG;
+  constexpr int NA = TA * KC / 1024, NB = TB * KC / 1024;  // float4s of A and of B per thread and stage
+  typedef float veca __attribute__((ext_vector_type(TM)));
+  typedef float vecb __attribute__((ext_vector_type(TN)));
+  __shared__ __align__(16) float As[2][KC][TA + 4], Bs[2][KC][TB + 4];
+  const uint32_t t = threadIdx.x, tx = t & 15, ty = t >> 4;
+  const uint32_t nt = (N + TB - 1) / TB, m0 = blockIdx.x / nt * TA, n0 = blockIdx.x % nt * TB;
+  float4 ra[NA], rb[NB];
+  // four k of one row of a [rows x K] matrix (zeros past K, some row's past the last)
+  auto row4 = [&](const float *p, uint32_t r, uint32_t rows, uint32_t k) {
+    const float *q = p + (size_t)(r < rows ? r : rows - 1) * K;
+    float4 v;
+    if (VEC) {
+      v = *(const float4 *)(q + (k < K ? k : K - 4));
+      if (k >= K) v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    } else {
+      v.x = k < K ? q[k] : 0.0f;
+      v.y = k + 1 < K ? q[k + 1] : 0.0f;
+      v.z = k + 2 < K ? q[k + 2] : 0.0f;
+      v.w = k + 3 < K ? q[k + 3] : 0.0f;
+    }
+    return v;
+  };
+  auto load = [&](uint32_t k0) {
+#pragma unroll
+    for (int j = 0; j < NA; j++) {
+      const uint32_t e = t + 256 * j;
+      ra[j] = row4(A, m0 + e % TA, M, k0 + 4 * (e / TA));
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      const uint32_t e = t + 256 * j;
+      if (TRANS_B) {
+        rb[j] = row4(B, n0 + e % TB, N, k0 + 4 * (e / TB));
+      } else {
+        const uint32_t k = k0 + e / (TB / 4), c = n0 + 4 * (e % (TB / 4));
+        const float *q = B + (size_t)(k < K ? k : K - 1) * N;
+        float4 v;
+        if (VEC) {
+          v = *(const float4 *)(q + (c < N ? c : N - 4));
+        } else {
+          v.x = q[c < N ? c : N - 1];
+          v.y = q[c + 1 < N ? c + 1 : N - 1];
+          v.z = q[c + 2 < N ? c + 2 : N - 1];
+          v.w = q[c + 3 < N ? c + 3 : N - 1];
+        }
+        rb[j] = k < K ? v : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < NA; j++) {
+      const uint32_t e = t + 256 * j, r = e % TA, k = 4 * (e / TA);
+      As[buf][k][r] = ra[j].x; As[buf][k + 1][r] = ra[j].y; As[buf][k + 2][r] = ra[j].z; As[buf][k + 3][r] = ra[j].w;
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+      const uint32_t e = t + 256 * j, r = e % TB, k = 4 * (e / TB);
+      if (TRANS_B) {
+        Bs[buf][k][r] = rb[j].x; Bs[buf][k + 1][r] = rb[j].y; Bs[buf][k + 2][r] = rb[j].z; Bs[buf][k + 3][r] = rb[j].w;
+      } else {
+        *(float4 *)&Bs[buf][e / (TB / 4)][4 * (e % (TB / 4))] = rb[j];
+      }
+    }
+  };
+  float acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const uint32_t c = n0 + TN * tx + j;
+      acc[i][j] = BIAS ? bias[c < N ? c : N - 1] : 0.0f;
+    }
+  struct KV {
+    veca a;
+    vecb b;
+  };
+  auto get = [&](int buf, int k) {
+    return KV{*(const veca *)&As[buf][k][TM * ty], *(const vecb *)&Bs[buf][k][TN * tx]};
+  };
+  load(0);
+  int buf = 0;
+  for (uint32_t k0 = 0; k0 < K; k0 += KC, buf ^= 1) {
+    const uint32_t kc = K - k0 < (uint32_t)KC ? K - k0 : (uint32_t)KC;
+    put(buf);
+    __syncthreads();  // the other buffer's readers passed the previous one
+    if (k0 + KC < K) load(k0 + KC);
+    if (ORDER == MM_SERIAL) {
+      if (kc == (uint32_t)KC) {
+        KV cur[KG], nxt[KG];
+#pragma unroll
+        for (int k = 0; k < KG; k++) cur[k] = get(buf, k);
+#pragma unroll
+        for (int kg = 0; kg < KC; kg += KG) {
+          if (kg + KG < KC) {
+#pragma unroll
+            for (int k = 0; k < KG; k++) nxt[k] = get(buf, kg + KG + k);
+          }
+          __builtin_amdgcn_sched_barrier(0);  // keep this order: reads, then the arithmetic
+#pragma unroll
+          for (int k = 0; k < KG; k++)
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+              for (int j = 0; j < TN; j++) acc[i][j] = __fadd_rn(acc[i][j], __fmul_rn(cur[k].a[i], cur[k].b[j]));
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int k = 0; k < KG; k++) cur[k] = nxt[k];
+        }
+      } else {
+        for (uint32_t k = 0; k < kc; k++) {
+          const KV v = get(buf, k);
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) acc[i][j] = __fadd_rn(acc[i][j], __fmul_rn(v.a[i], v.b[j]));
+        }
+      }
+    } else {
+      // kernels.el:99-104: acc + (p0 + (p1 + ... (p14 + p15))) per tile of 16, zero products past K
+      for (uint32_t kb = 0; kb < kc; kb += 16) {
+        float s[TM][TN];
+        KV cur = get(buf, kb + 15);
+#pragma unroll
+        for (int q = 15; q >= 0; q--) {
+          KV nxt;
+          if (q) nxt = get(buf, kb + q - 1);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++) {
+              const float p = __fmul_rn(cur.a[i], cur.b[j]);
+              s[i][j] = q == 15 ? p : __fadd_rn(p, s[i][j]);
+            }
+          cur = nxt;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+          for (int j = 0; j < TN; j++) acc[i][j] = __fadd_rn(acc[i][j], s[i][j]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const uint32_t row = m0 + TM * ty + i, col = n0 + TN * tx + j;
+      if (row < M && col < N && mm_covered(row, col, N, lim_mode, lim)) C[(size_t)row * N + col] = acc[i][j];
+    }
 }
 
 template <int ORDER>
@@ -101,11 +274,44 @@ static void mm_go(const float *A, const float *B, const float *bias, float *C, u
   }
 }
 
+template <int TM, int TN, int ORDER, bool VEC>
+static void mmt_go(const float *A, const float *B, const float *bias, float *C, uint32_t M, uint32_t N, uint32_t K,
+                   bool trans_b, int lim_mode, uint64_t lim, hipStream_t st) {
+  constexpr uint32_t TA = 16 * TM, TB = 16 * TN;
+  const dim3 g((uint32_t)((uint64_t)((M + TA - 1) / TA) * ((N + TB - 1) / TB))), b(256);
+  if (!trans_b) hipLaunchKernelGGL((k_mmt<TM, TN, ORDER, false, false, VEC>), g, b, 0, st, A, B, bias, C, M, N, K, lim_mode, lim);
+  else if constexpr (ORDER == MM_SERIAL)
+    hipLaunchKernelGGL((k_mmt<TM, TN, ORDER, true, true, VEC>), g, b, 0, st, A, B, bias, C, M, N, K, lim_mode, lim);
+}
+
+template <int TM, int TN>
+static void mmt(const float *A, const float *B, const float *bias, float *C, uint32_t M, uint32_t N, uint32_t K,
+                bool trans_b, int order, int lim_mode, uint64_t lim, hipStream_t st) {
+  const bool vec = K % 4 == 0 && (trans_b || N % 4 == 0) && (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
+  if (order == MM_TILE16) {
+    if (vec) mmt_go<TM, TN, MM_TILE16, true>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
+    else mmt_go<TM, TN, MM_TILE16, false>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
+  } else {
+    if (vec) mmt_go<TM, TN, MM_SERIAL, true>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
+    else mmt_go<TM, TN, MM_SERIAL, false>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
+  }
+}
 static int mm(const float *A, const float *B, const float *bias, float *C, uint32_t M, uint32_t N, uint32_t K,
               bool trans_b, int order, int lim_mode, uint64_t lim, hipStream_t st, const char *name) {
   if (!M || !N || !lim) return NLG_OK;
   if (nlg_blocks(M, MM_T) > 65535) return nlg_fail("%s: M = %u is too large", name, M);
-  if (order == MM_TILE16) mm_go<MM_TILE16>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
+  auto tiles = [&](uint64_t ta, uint64_t tb) { return ((M + ta - 1) / ta) * ((N + tb - 1) / tb); };
+  const uint64_t cu = nlg_num_cu();
+  // Larger tiles read less per product but need several workgroups per CU to
+  // issue at the full rate.  us with 64 x 64 / 64 x 32 / 32 x 32 / 16 x 16 tiles:
+  // 2,048^3 349 / 380 / 509 / 1,024; 1,536 x 1,024 x 1,536 (576 / 1,152 / 2,304
+  // tiles) 137 / 121 / 148 / 291; 1,024^3 81 / 56 / 71 / 133; 768^3 (144 / 288 /
+  // 576) 61 / 42 / 43 / 60; 512^3 42 / 26 / 16 / 20; 384^3 (36 / 72 / 144) 32 / 20 /
+  // 12.4 / 13.9; 64 x 2,048 x 2,048 (128 tiles of 32 x 32) 157 / 95 / 57 / 42.
+  if (K && tiles(64, 64) >= 3 * cu) mmt<4, 4>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
+  else if (K && tiles(64, 32) >= cu) mmt<4, 2>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
+  else if (K && tiles(32, 32) >= cu * 3 / 4) mmt<2, 2>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
+  else if (order == MM_TILE16) mm_go<MM_TILE16>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
   else mm_go<MM_SERIAL>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
   NLG_LAUNCHED(name);
   return NLG_OK;
