@@ -15,11 +15,15 @@
 
 // The reference's max starts from the first element and only moves on a
 // strict `>`: NaNs are never selected, except that a NaN first element stays.
-template <int EPT, bool V4>
-__global__ __launch_bounds__(256) void k_softmax_reg(const float *a, float *c, uint32_t rows,
-                                                     uint32_t n) {
-  __shared__ float red[4];
-  const uint32_t row = blockIdx.x;
+// TPR threads take a row and hold EPT of its values each: a wave (no LDS, no
+// barrier; four rows a workgroup), a workgroup of 256 or one of 1,024.
+template <int TPR, int EPT, bool V4>
+__global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void k_softmax_reg(const float *a, float *c, uint32_t rows,
+                                                                      uint32_t n) {
+  __shared__ float red[TPR < 256 ? 1 : TPR / 64];
+  constexpr bool WAVE = TPR == 64;
+  const uint32_t tid = threadIdx.x % TPR;
+  const uint32_t row = WAVE ? blockIdx.x * 4 + threadIdx.x / 64 : blockIdx.x;
   if (row >= rows) return;
   const float *ar = a + (size_t)row * n;
   float *cr = c + (size_t)row * n;
@@ -29,7 +33,7 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const float *a, float *c, u
   if (V4) {
 #pragma unroll
     for (int k = 0; k < EPT / 4; k++) {
-      const uint32_t i4 = threadIdx.x + 256u * k;
+      const uint32_t i4 = tid + TPR * k;
       float4 q = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
       if (4 * i4 < n) q = nlg_ld_stream_f4((const float4 *)ar + i4);
       v[4 * k] = q.x; v[4 * k + 1] = q.y; v[4 * k + 2] = q.z; v[4 * k + 3] = q.w;
@@ -37,26 +41,26 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const float *a, float *c, u
   } else {
 #pragma unroll
     for (int k = 0; k < EPT; k++) {
-      const uint32_t i = threadIdx.x + 256u * k;
+      const uint32_t i = tid + TPR * k;
       v[k] = i < n ? ar[i] : -INFINITY;
     }
   }
 #pragma unroll
   for (int k = 0; k < EPT; k++) mx = v[k] > mx ? v[k] : mx;
-  mx = nlg_block_max_f32(mx, red);
+  mx = WAVE ? nlg_wave_max_f32(mx) : nlg_block_max_f32(mx, red);
   if (first != first) mx = first;
   float s = 0.0f;
 #pragma unroll
   for (int k = 0; k < EPT; k++) {
-    const uint32_t i = V4 ? 4 * (threadIdx.x + 256u * (k / 4)) + (k % 4) : threadIdx.x + 256u * k;
+    const uint32_t i = V4 ? 4 * (tid + TPR * (k / 4)) + (k % 4) : tid + TPR * k;
     v[k] = expf(__fsub_rn(v[k], mx));
     if (i < n) s = __fadd_rn(s, v[k]);
   }
-  s = nlg_block_sum_f32(s, red);
+  s = WAVE ? nlg_wave_sum_f32(s) : nlg_block_sum_f32(s, red);
   if (V4) {
 #pragma unroll
     for (int k = 0; k < EPT / 4; k++) {
-      const uint32_t i4 = threadIdx.x + 256u * k;
+      const uint32_t i4 = tid + TPR * k;
       if (4 * i4 < n)
         nlg_st_stream_f4((float4 *)cr + i4,
                          make_float4(v[4 * k] / s, v[4 * k + 1] / s, v[4 * k + 2] / s, v[4 * k + 3] / s));
@@ -64,7 +68,7 @@ __global__ __launch_bounds__(256) void k_softmax_reg(const float *a, float *c, u
   } else {
 #pragma unroll
     for (int k = 0; k < EPT; k++) {
-      const uint32_t i = threadIdx.x + 256u * k;
+      const uint32_t i = tid + TPR * k;
       if (i < n) cr[i] = v[k] / s;
     }
   }
@@ -90,20 +94,26 @@ __global__ __launch_bounds__(256) void k_softmax_stream(const float *a, float *c
   for (uint32_t i = threadIdx.x; i < n; i += 256) cr[i] = expf(__fsub_rn(ar[i], mx)) / s;
 }
 
+#define SMW 1024
+
 static int launch_softmax(const float *a, float *c, uint32_t rows, uint32_t n, hipStream_t st) {
   if (!rows || !n) return NLG_OK;
   const bool v4 = (n % 4 == 0) && ((((uintptr_t)a) | ((uintptr_t)c)) & 15) == 0;
-  dim3 g(rows), b(256);
-#define SM(EPT)                                                                  \
-  do {                                                                           \
-    if (v4) hipLaunchKernelGGL((k_softmax_reg<EPT, true>), g, b, 0, st, a, c, rows, n); \
-    else hipLaunchKernelGGL((k_softmax_reg<EPT, false>), g, b, 0, st, a, c, rows, n);   \
+#define SM(TPR, EPT)                                                                                   \
+  do {                                                                                                 \
+    const dim3 g(TPR == 64 ? (rows + 3) / 4 : rows), b(TPR == 64 ? 256 : TPR);                         \
+    if (v4) hipLaunchKernelGGL((k_softmax_reg<TPR, EPT, true>), g, b, 0, st, a, c, rows, n);           \
+    else hipLaunchKernelGGL((k_softmax_reg<TPR, EPT, false>), g, b, 0, st, a, c, rows, n);             \
   } while (0)
-  if (n <= 256 * 4) SM(4);
-  else if (n <= 256 * 8) SM(8);
-  else if (n <= 256 * 16) SM(16);
-  else if (n <= 256 * 32) SM(32);
-  else hipLaunchKernelGGL(k_softmax_stream, g, b, 0, st, a, c, rows, n);
+  if (n <= 64 * 4) SM(64, 4);
+  else if (n <= SMW) SM(64, 16);
+  else if (n <= 256 * 4) SM(256, 4);
+  else if (n <= 256 * 8) SM(256, 8);
+  else if (n <= 256 * 16) SM(256, 16);
+  else if (n <= 256 * 32) SM(256, 32);
+  else if (n <= 1024 * 16) SM(1024, 16);
+  else if (n <= 1024 * 32) SM(1024, 32);
+  else hipLaunchKernelGGL(k_softmax_stream, dim3(rows), dim3(256), 0, st, a, c, rows, n);
 #undef SM
   NLG_LAUNCHED("softmax");
   return NLG_OK;

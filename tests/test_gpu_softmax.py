@@ -53,3 +53,33 @@ def test_softmax_matches_oracle(heads, n, inplace):
         assert rel_exact.max() <= 1e-5, rel_exact.max()
     sums = got.reshape(rows, n).astype(np.float64).sum(axis=1)
     assert np.abs(sums - 1).max() < 1e-4
+
+
+@pytest.mark.parametrize("n", [1, 3, 63, 64, 65, 255, 256, 257, 260, 511, 1000, 1023, 1024, 1025, 1028, 8192, 8193,
+                               8196, 16384, 16385, 16388, 20001, 32767, 32768, 32769])
+@pytest.mark.parametrize("inplace", [False, True])
+def test_softmax_row_widths(n, inplace):
+    """Edges of the forms a row takes (a wave, 256 threads, 1,024 threads, three
+    passes) and of their whole-float4 variants; rows that start with a NaN, hold
+    one, are all -inf, or hold +inf end as the reference's."""
+    rows = 11
+    print(f"[gpu] softmax rows={rows} n={n} inplace={inplace}", flush=True)
+    a = nlgpu.normal(n, rows * n, 3.0).reshape(rows, n)
+    a[3] = -np.inf
+    a[4, 0] = np.nan
+    a[5, n // 2] = np.inf
+    a[6, n - 1] = np.nan
+    a[7, :] = np.finfo(np.float32).min
+    a = a.ravel()
+    da = nlgpu.to_device(a)
+    dc = da if inplace else nlgpu.DeviceArray(a.nbytes)
+    nlgpu.softmax_rows(da, dc, rows, n)
+    got = dc.download(np.float32, rows * n).reshape(rows, n)
+    with np.errstate(all="ignore"):
+        want = orc.softmax_rows(a, rows, n).reshape(rows, n)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    x = a.reshape(rows, n).astype(np.float64)
+    live = [r for r in range(rows) if not np.isnan(want[r]).any()]
+    e = np.exp(x[live] - x[live].max(axis=1, keepdims=True))
+    exact = e / e.sum(axis=1, keepdims=True)
+    assert np.max(np.abs(got[live] - exact) / exact) <= 1e-5
