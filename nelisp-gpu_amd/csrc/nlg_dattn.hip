@@ -54,8 +54,8 @@ struct AttnArgs {
 };
 
 // how k_attn_part finds position p's K/V row; AM_NT added to a mode: K and V
-// read with non-temporal loads
-enum { AM_CONTIG = 0, AM_PAGED = 1, AM_RING = 2, AM_ENTRIES = 3, AM_NT = 8 };
+// read with non-temporal loads; AM_LOOP: a workgroup takes several chunks
+enum { AM_CONTIG = 0, AM_PAGED = 1, AM_RING = 2, AM_ENTRIES = 3, AM_NT = 8, AM_LOOP = 16 };
 
 // K/V row loads, plain or non-temporal
 template <bool NT>
@@ -121,10 +121,35 @@ __device__ __forceinline__ float4 keep_f4(bool ok, float4 v) {
   return make_float4(ok ? v.x : 0.0f, ok ? v.y : 0.0f, ok ? v.z : 0.0f, ok ? v.w : 0.0f);
 }
 
+// The partials of a chunk past the position: no weight, marked by a sum of -0
+// (a sum of exponentials never is).  Past ATTN_MERGE_ALL chunks the merge skips
+// such a chunk's context, which is then not written either; up to it, the merges
+// (the output projection's among them) read every chunk's.
+#define ATTN_MERGE_ALL 12
+static_assert(NLG_ATTN_MAX_CHUNKS <= ATTN_MERGE_ALL, "the output projection reads every chunk");
+template <int HD, int G>
+__device__ __forceinline__ void attn_no_chunk(const AttnArgs &a, float *pctx, float *pmz) {
+  if (a.nchunk <= ATTN_MERGE_ALL)
+    for (int i = threadIdx.x; i < G * HD; i += ATTN_WAVES * 64) pctx[i] = 0.0f;
+  if (threadIdx.x < G) {
+    pmz[2 * threadIdx.x] = -1.0e30f;
+    pmz[2 * threadIdx.x + 1] = -0.0f;
+  }
+}
+// The chunks c, c + step, ... of a (query row, head group) unit, all past the
+// position.
+template <int HD, int G>
+__device__ __forceinline__ void attn_no_chunks(const AttnArgs &a, uint32_t qr, uint32_t h0, uint32_t c, uint32_t step) {
+  for (; c < a.nchunk; c += step) {
+    const size_t cb = (size_t)qr * a.nchunk + c;
+    attn_no_chunk<HD, G>(a, a.pctx + cb * a.heads * HD + (size_t)h0 * HD, a.pmz + (cb * a.heads + h0) * 2);
+  }
+}
+
 template <int HD, int G, int NI, int MODE>
 __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
-  constexpr int BM = MODE & ~AM_NT;
-  constexpr bool NT = (MODE & AM_NT) != 0;
+  constexpr int BM = MODE & 7;
+  constexpr bool NT = (MODE & AM_NT) != 0, LOOP = (MODE & AM_LOOP) != 0;
   constexpr bool PG = BM == AM_PAGED, RG = BM == AM_RING || BM == AM_ENTRIES, EN = BM == AM_ENTRIES;
   constexpr int LPP = HD / 8, PPI = 64 / LPP, PW = NI * PPI, NW = ATTN_WAVES, CS = NW * PW;
   __shared__ float s_m[NW][G], s_z[NW][G];
@@ -150,6 +175,16 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   }
   const uint32_t kvh = h0 / a.grp;
   const uint32_t b = a.qper ? qr / a.qper : qr;                         // its sequence
+  // AM_LOOP (large caches, whose position is in hand first): the workgroup takes
+  // chunks blockIdx.x, + gridDim.x, ... and stops at the first past the position,
+  // so room for a longer context costs no workgroups that find nothing to do
+  // (each holds a slot for two round trips: 8 sequences at position 4,095, 8 kv
+  // heads, 39.3 us with room for 8,192 positions, 28.3 with 4,096; now 31.2).
+  static_assert(!LOOP || (NT && !RG && G > 1), "a loop needs the position first");
+  for (;; c += gridDim.x) {
+  // (q again for each chunk: held over the loop it costs the second workgroup
+  // of a CU its registers)
+  if (LOOP) asm volatile("" ::: "memory");
   const size_t cb = (size_t)qr * a.nchunk + c;
   float *pctx = a.pctx + cb * a.heads * HD + (size_t)h0 * HD;
   float *pmz = a.pmz + (cb * a.heads + h0) * 2;
@@ -191,6 +226,11 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   if (NT && !RG) {
     const int32_t pr = PG ? (a.lens ? a.lens[b] : a.pos[0]) : a.pos[0] + (a.qper ? (int32_t)(qr % a.qper) : 0);
     lim = (pr < 0 ? 0u : ((uint32_t)pr >= a.max_seq ? a.max_seq - 1 : (uint32_t)pr)) + 1;
+    if (p0 >= lim) {  // block-uniform
+      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, gridDim.x);
+      else attn_no_chunk<HD, G>(a, pctx, pmz);
+      return;
+    }
   }
   if (EN) {
     // the list entries first, then the rows and rotations they name
@@ -294,11 +334,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
     len = (pr < 0 ? 0u : ((uint32_t)pr >= a.max_seq ? a.max_seq - 1 : (uint32_t)pr)) + 1;
   }
   if (p0 >= len) {  // block-uniform: a chunk past the position adds nothing
-    for (int i = threadIdx.x; i < G * HD; i += NW * 64) pctx[i] = 0.0f;
-    if (threadIdx.x < G) {
-      pmz[2 * threadIdx.x] = -1.0e30f;
-      pmz[2 * threadIdx.x + 1] = 0.0f;
-    }
+    attn_no_chunk<HD, G>(a, pctx, pmz);
     return;
   }
   float s[NI][G];
@@ -391,6 +427,9 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
       pmz[2 * h + 1] = zz;
     }
   }
+  if (!LOOP || c + gridDim.x >= a.nchunk) return;
+  __syncthreads();  // the waves' partials have been read
+  }
 }
 
 // The chunk pass on the matrix cores, for head_dim 128, 4 query heads per
@@ -421,7 +460,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
 // reductions and conversions; here they are 32 matrix-core steps per wave.
 #define AMF_PITCH 36  // V^T tile row pitch in 16-bit elements (32 slots + 4: 8-byte aligned rows)
 
-template <bool NT, bool RG>
+template <bool NT, bool RG, bool LOOP = false>
 __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
   constexpr int HD = 128, G = 4, NW = ATTN_WAVES, PW = 32, CS = NW * PW;
   typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -433,13 +472,10 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
                "s"(a.kvheads), "s"(a.max_seq), "s"(a.nchunk), "s"(a.coef));
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  const uint32_t c = blockIdx.x, h0 = blockIdx.y * G, qr = blockIdx.z;
+  uint32_t c = blockIdx.x;
+  const uint32_t h0 = blockIdx.y * G, qr = blockIdx.z;
   const uint32_t kvh = h0 / a.grp;
   const uint32_t b = a.qper ? qr / a.qper : qr;  // its sequence
-  const size_t cb = (size_t)qr * a.nchunk + c;
-  float *pctx = a.pctx + cb * a.heads * HD + (size_t)h0 * HD;
-  float *pmz = a.pmz + (cb * a.heads + h0) * 2;
-  const uint32_t p0 = c * CS, pw = p0 + w * PW;
   const size_t slot = (size_t)b * a.kvheads + kvh;
   const uint16_t *kb = a.kc + slot * a.max_seq * HD;
   const uint16_t *vb = a.vc + slot * a.max_seq * HD;
@@ -459,6 +495,13 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
     const uint32_t t = woff + (pc - a.nsink);  // < 2 win
     return a.nsink + (t >= a.win ? t - a.win : t);
   };
+  static_assert(!LOOP || (NT && !RG), "a loop needs the position first");
+  for (;; c += gridDim.x) {  // LOOP: as in k_attn_part
+  if (LOOP) asm volatile("" ::: "memory");
+  const size_t cb = (size_t)qr * a.nchunk + c;
+  float *pctx = a.pctx + cb * a.heads * HD + (size_t)h0 * HD;
+  float *pmz = a.pmz + (cb * a.heads + h0) * 2;
+  const uint32_t p0 = c * CS, pw = p0 + w * PW;
   // q first (loads retire in issue order): lane (lg, li) takes head
   // h0 + li (li < 4; the others zero), dims 32 s + 8 lg .. + 7
   const float *qb = a.q + (size_t)qr * a.heads * HD + (size_t)(h0 + (li < G ? li : 0)) * HD + 8 * lg;
@@ -477,6 +520,11 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
     const int32_t pr = a.pos[0] + (a.qper ? (int32_t)(qr % a.qper) : 0);
     lim = (pr < 0 ? 0u : ((uint32_t)pr >= a.max_seq ? a.max_seq - 1 : (uint32_t)pr)) + 1;
     len = lim;  // positions attended: 0 .. pr
+    if (p0 >= lim) {  // block-uniform
+      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, gridDim.x);
+      else attn_no_chunk<HD, G>(a, pctx, pmz);
+      return;
+    }
   }
   // K rows of the wave's 32 positions go straight into its tile (direct
   // global-to-LDS loads, whole rows per instruction: instruction k, lane
@@ -545,11 +593,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
   if (p0 >= len) {  // block-uniform: a chunk past the position adds nothing
     // (the tile's direct loads land before the workgroup's LDS is released)
     if (KLDS) __builtin_amdgcn_s_waitcnt(0);
-    for (int i = threadIdx.x; i < G * HD; i += NW * 64) pctx[i] = 0.0f;
-    if (threadIdx.x < G) {
-      pmz[2 * threadIdx.x] = -1.0e30f;
-      pmz[2 * threadIdx.x + 1] = 0.0f;
-    }
+    attn_no_chunk<HD, G>(a, pctx, pmz);
     return;
   }
   v8h qh[4], ql[4];
@@ -708,6 +752,9 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       pmz[2 * h + 1] = zz;
     }
   }
+  if (!LOOP || c + gridDim.x >= a.nchunk) return;
+  __syncthreads();  // the waves' contexts have been read
+  }
 }
 
 // Pass 2: out = sum_c pctx_c * exp(m_c - M) / sum_c z_c * exp(m_c - M),
@@ -755,6 +802,78 @@ __global__ __launch_bounds__(256) void k_attn_merge(const float *__restrict__ pc
   out[i] = acc / zz;
 }
 
+// The same over many chunks, a workgroup of hd threads per (row, head): the
+// chunks' weights are computed once, by all threads, into LDS instead of by
+// every thread from its own loads, and the contexts of chunks past the position
+// (a suffix, marked by a sum of -0) are not read.  The sums run in k_attn_merge's
+// order: the same bits.
+#define MERGE_TILE 512
+__global__ void k_attn_merge_many(const float *__restrict__ pctx, const float *__restrict__ pmz,
+                                  float *__restrict__ out, uint32_t heads, uint32_t hd, uint32_t nchunk) {
+  __shared__ float s_sc[MERGE_TILE], s_z[MERGE_TILE], s_m[2];
+  __shared__ uint32_t s_n[2];
+  const uint32_t b = blockIdx.x / heads, h = blockIdx.x % heads, t = threadIdx.x, w = t >> 6;
+  const float *mz = pmz + ((size_t)b * nchunk * heads + h) * 2;
+  float mm = -1.0e30f;
+  uint32_t live = 0;  // chunks up to the last with a weight
+  for (uint32_t c = t; c < nchunk; c += hd) {
+    const float2 v = *(const float2 *)(mz + (size_t)c * heads * 2);
+    mm = v.x > mm ? v.x : mm;
+    if (__float_as_uint(v.y) != 0x80000000u) live = c + 1;
+  }
+  mm = nlg_wave_max_f32(mm);
+  for (int off = 32; off; off >>= 1) {
+    const uint32_t o = __shfl_xor(live, off);
+    live = o > live ? o : live;
+  }
+  if ((t & 63) == 0) {
+    s_m[w] = mm;
+    s_n[w] = live;
+  }
+  __syncthreads();
+  if (hd > 64) {
+    mm = s_m[0] > s_m[1] ? s_m[0] : s_m[1];
+    live = s_n[0] > s_n[1] ? s_n[0] : s_n[1];
+  }
+  const float *cx = pctx + (size_t)b * nchunk * heads * hd + (size_t)h * hd + t;
+  const size_t cs = (size_t)heads * hd;
+  float zz = 0.0f, acc = 0.0f;
+  for (uint32_t c0 = 0; c0 < live; c0 += MERGE_TILE) {
+    const uint32_t n = live - c0 < MERGE_TILE ? live - c0 : MERGE_TILE;
+    if (c0) __syncthreads();
+    for (uint32_t c = t; c < n; c += hd) {
+      const float2 v = *(const float2 *)(mz + (size_t)(c0 + c) * heads * 2);
+      s_sc[c] = nlg_exp2(v.x - mm);
+      s_z[c] = v.y;
+    }
+    __syncthreads();
+    for (uint32_t c = 0; c < n; c += 8) {
+      float x[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) x[k] = cx[(c0 + (c + k < n ? c + k : n - 1)) * cs];
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (c + k < n) {
+          zz = fmaf(s_z[c + k], s_sc[c + k], zz);
+          acc = fmaf(x[k], s_sc[c + k], acc);
+        }
+    }
+  }
+  out[((size_t)b * heads + h) * hd + t] = acc / zz;
+}
+
+// At 10 chunks (one sequence, 20 heads) k_attn_merge is 0.3 us ahead; at 17 / 19 /
+// 32 / 125 this form is, by 0.5 / 0.7 / 1.6 / 7 us.
+static void attn_merge_launch(const AttnArgs &a, float *out, uint32_t rows, uint32_t hd, hipStream_t st) {
+  const uint64_t n = (uint64_t)rows * a.heads * hd;
+  if (a.nchunk > ATTN_MERGE_ALL)
+    hipLaunchKernelGGL(k_attn_merge_many, dim3(rows * a.heads), dim3(hd), 0, st, a.pctx, a.pmz, out, a.heads, hd,
+                       a.nchunk);
+  else
+    hipLaunchKernelGGL(k_attn_merge, dim3(nlg_blocks(n, 256)), dim3(256), 0, st, a.pctx, a.pmz, out, rows, a.heads,
+                       hd, a.nchunk);
+}
+
 extern "C" size_t nlg_decode_attn_f16_workspace(uint32_t batch, uint32_t heads, uint32_t kvheads,
                                                 uint32_t head_dim, uint32_t max_seq) {
   if (!kvheads || (head_dim != 64 && head_dim != 128) || !max_seq) return 0;
@@ -798,17 +917,35 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
   if (mode != AM_ENTRIES && seqs * a.kvheads * a.max_seq * head_dim * 4 >= ATTN_NT_BYTES) mode |= AM_NT;
   constexpr int AM_CONTIG_NT_ = AM_CONTIG | AM_NT;
   a.nunits = rows * a.kvheads * a.nchunk;
-  const dim3 grid = G == 1 ? dim3((a.nunits + 7) / 8 * 8 * a.grp) : dim3(a.nchunk, a.heads / G, rows);
+  // Many chunks of a large cache: workgroups that loop over their unit's, four
+  // per CU over contiguous caches (all at one position), eight over paged ones
+  // (lengths differ, so they need more to balance).  us with 2 / 4 / 8 per CU:
+  // 8 sequences at 4,095 of 8,192, 8 kv heads 30.7 / 31.2 / 37.6 (39.3 one chunk
+  // each); 32 paged ones of up to 4,096, 5 kv heads 66 / 58 / 51.5 (60.7).  Of few
+  // chunks few are past the position and the loop only unbalances: 46 sequences,
+  // 8 kv heads, 5 chunks 38.4 / 40.8 / 36.3 (34.9).
+  const uint64_t units = (uint64_t)rows * (a.heads / G);
+  const int bm0 = mode & 7;
+  uint32_t gx = a.nchunk;
+  if (G > 1 && (mode & AM_NT) && (bm0 == AM_CONTIG || bm0 == AM_PAGED) && a.nchunk >= 8) {
+    const uint64_t want = ((bm0 == AM_PAGED ? 8ull : 4ull) * nlg_num_cu() + units - 1) / units;
+    if (want < gx) {
+      gx = (uint32_t)want;
+      mode |= AM_LOOP;
+    }
+  }
+  const dim3 grid = G == 1 ? dim3((a.nunits + 7) / 8 * 8 * a.grp) : dim3(gx, a.heads / G, rows);
   const dim3 blk(ATTN_WAVES * 64);
   // (ring caches small enough for plain loads keep the VALU pass: that
   // variant's registers spill under the two-workgroups-per-CU bound)
   if (head_dim == 128 && G == 4 && ni == 8 &&
-      ((mode & ~AM_NT) == AM_CONTIG || mode == (AM_RING | AM_NT))) {
-    const bool nt = mode & AM_NT, rg = (mode & ~AM_NT) == AM_RING;
+      (bm0 == AM_CONTIG || mode == (AM_RING | AM_NT))) {
+    const bool nt = mode & AM_NT, rg = bm0 == AM_RING;
     if (rg) {
       hipLaunchKernelGGL((k_attn_mfma<true, true>), grid, blk, 0, st, a);
     } else {
-      if (nt) hipLaunchKernelGGL((k_attn_mfma<true, false>), grid, blk, 0, st, a);
+      if (mode & AM_LOOP) hipLaunchKernelGGL((k_attn_mfma<true, false, true>), grid, blk, 0, st, a);
+      else if (nt) hipLaunchKernelGGL((k_attn_mfma<true, false>), grid, blk, 0, st, a);
       else hipLaunchKernelGGL((k_attn_mfma<false, false>), grid, blk, 0, st, a);
     }
     NLG_LAUNCHED(rg ? "decode attention (ring fp16 KV, matrix cores)" : "decode attention (fp16 KV, matrix cores)");
@@ -819,9 +956,17 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
     if (ni == 8) hipLaunchKernelGGL((k_attn_part<HD, GG, 8, PGV>), grid, blk, 0, st, a);   \
     else hipLaunchKernelGGL((k_attn_part<HD, GG, 4, PGV>), grid, blk, 0, st, a);           \
   } while (0)
+// (a loop: ni is 8 at 8 chunks and more, G at least 2)
 #define AT(HD, GG)                                                                         \
   do {                                                                                     \
-    if (mode == AM_PAGED) AT1(HD, GG, AM_PAGED);                                           \
+    if (mode & AM_LOOP) {                                                                  \
+      if constexpr (GG > 1) {                                                              \
+        if (bm0 == AM_PAGED)                                                               \
+          hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_PAGED | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
+        else if constexpr (HD != 128 || GG != 4) /* those: matrix cores */                 \
+          hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_CONTIG | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
+      }                                                                                    \
+    } else if (mode == AM_PAGED) AT1(HD, GG, AM_PAGED);                                           \
     else if (mode == (AM_PAGED | AM_NT)) AT1(HD, GG, AM_PAGED | AM_NT);                    \
     else if (mode == AM_RING) AT1(HD, GG, AM_RING);                                        \
     else if (mode == (AM_RING | AM_NT)) AT1(HD, GG, AM_RING | AM_NT);                      \
@@ -836,7 +981,7 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
   }
 #undef AT
 #undef AT1
-  const int bm = mode & ~AM_NT;
+  const int bm = bm0;
   NLG_LAUNCHED(bm == AM_PAGED     ? "decode attention (paged fp16 KV)"
                : bm == AM_RING    ? "decode attention (ring fp16 KV)"
                : bm == AM_ENTRIES ? "decode attention (fp16 KV entry list)"
@@ -914,9 +1059,7 @@ extern "C" int nlg_decode_attn_paged_f16(const float *q, const uint16_t *kpool, 
   a.table = table; a.lens = lens; a.bs = bs; a.mbps = mbps; a.npool = npool;
   hipStream_t st = nlg_stream(stream);
   if (attn_chunks_launch(a, batch, head_dim, AM_PAGED, st)) return NLG_ERR;
-  const uint64_t n = (uint64_t)batch * heads * head_dim;
-  hipLaunchKernelGGL(k_attn_merge, dim3(nlg_blocks(n, 256)), dim3(256), 0, st, a.pctx, a.pmz, out, batch,
-                     heads, head_dim, a.nchunk);
+  attn_merge_launch(a, out, batch, head_dim, st);
   NLG_LAUNCHED("paged decode attention merge");
   return NLG_OK;
 }
@@ -980,9 +1123,7 @@ extern "C" int nlg_decode_attn_stream_f16(const float *q, const uint16_t *kcache
   a.co = co; a.si = si; a.nsink = nsink; a.win = win;
   hipStream_t st = nlg_stream(stream);
   if (attn_chunks_launch(a, batch, head_dim, AM_RING, st)) return NLG_ERR;
-  const uint64_t n = (uint64_t)batch * heads * head_dim;
-  hipLaunchKernelGGL(k_attn_merge, dim3(nlg_blocks(n, 256)), dim3(256), 0, st, a.pctx, a.pmz, out, batch,
-                     heads, head_dim, a.nchunk);
+  attn_merge_launch(a, out, batch, head_dim, st);
   NLG_LAUNCHED("ring decode attention merge");
   return NLG_OK;
 }
@@ -1014,9 +1155,7 @@ extern "C" int nlg_attn_entries_f16(const float *q, const uint16_t *kcache, cons
   a.co = co; a.si = si; a.ent = ent; a.nslots = nslots; a.trows = trows;
   hipStream_t st = nlg_stream(stream);
   if (attn_chunks_launch(a, batch, head_dim, AM_ENTRIES, st)) return NLG_ERR;
-  const uint64_t n = (uint64_t)batch * heads * head_dim;
-  hipLaunchKernelGGL(k_attn_merge, dim3(nlg_blocks(n, 256)), dim3(256), 0, st, a.pctx, a.pmz, out, batch,
-                     heads, head_dim, a.nchunk);
+  attn_merge_launch(a, out, batch, head_dim, st);
   NLG_LAUNCHED("entry-list decode attention merge");
   return NLG_OK;
 }
@@ -1107,9 +1246,7 @@ extern "C" int nlg_decode_attn_f16(const float *q, const uint16_t *kcache, const
   AttnArgs a;
   attn_setup(a, batch, heads, kvheads, head_dim, max_seq, workspace, workspace_bytes);
   hipStream_t st = nlg_stream(stream);
-  const uint64_t n = (uint64_t)batch * heads * head_dim;
-  hipLaunchKernelGGL(k_attn_merge, dim3(nlg_blocks(n, 256)), dim3(256), 0, st, a.pctx, a.pmz, out, batch,
-                     heads, head_dim, a.nchunk);
+  attn_merge_launch(a, out, batch, head_dim, st);
   NLG_LAUNCHED("decode attention merge");
   return NLG_OK;
 }
