@@ -48,9 +48,10 @@ struct AttnArgs {
   // [0, trows) as zero rotations
   const int32_t *ent;
   uint32_t nslots, trows;
-  // one query head per workgroup (G == 1): units (row, kv head, chunk) on a
-  // 1-D grid, the grp workgroups of a unit on one XCD (see attn_unit)
+  // workgroups of fewer than grp query heads (nunits not 0): units (row, kv
+  // head, first chunk) on a 1-D grid, a unit's grp / G workgroups on one XCD
   uint32_t nunits;
+  uint32_t cstep;  // first chunks per (row, kv head): a looping workgroup's step
 };
 
 // how k_attn_part finds position p's K/V row; AM_NT added to a mode: K and V
@@ -159,16 +160,17 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // workgroup: chunk c, query heads h0 .. h0+G-1 (all of one kv head), query row qr
   uint32_t c, h0, qr;
-  if (G == 1) {
+  if (G == 1 || (G == 4 && !LOOP && !RG && a.nunits)) {
     // Workgroups are dealt to the 8 XCDs round-robin by id, and each XCD
-    // has its own L2: the grp query heads of one (row, kv head, chunk) unit
-    // get ids u%8 + 8(q + grp*(u/8)), all on XCD u%8, so the unit's K/V rows
+    // has its own L2: the n = grp / G workgroups of one (row, kv head, chunk)
+    // unit get ids u%8 + 8(q + n*(u/8)), all on XCD u%8, so the unit's K/V rows
     // come from HBM once and from that L2 for the other heads.
-    const uint32_t id = blockIdx.x, rest = id >> 3, q = rest % a.grp, u = (id & 7u) + 8u * (rest / a.grp);
+    const uint32_t n = a.grp / G;
+    const uint32_t id = blockIdx.x, rest = id >> 3, q = rest % n, u = (id & 7u) + 8u * (rest / n);
     if (u >= a.nunits) return;
-    c = u % a.nchunk;
-    const uint32_t r2 = u / a.nchunk;
-    h0 = (r2 % a.kvheads) * a.grp + q;
+    c = u % a.cstep;
+    const uint32_t r2 = u / a.cstep;
+    h0 = (r2 % a.kvheads) * a.grp + q * G;
     qr = r2 / a.kvheads;
   } else {
     c = blockIdx.x; h0 = blockIdx.y * G; qr = blockIdx.z;
@@ -176,12 +178,12 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   const uint32_t kvh = h0 / a.grp;
   const uint32_t b = a.qper ? qr / a.qper : qr;                         // its sequence
   // AM_LOOP (large caches, whose position is in hand first): the workgroup takes
-  // chunks blockIdx.x, + gridDim.x, ... and stops at the first past the position,
+  // chunks c, c + cstep, ... and stops at the first past the position,
   // so room for a longer context costs no workgroups that find nothing to do
   // (each holds a slot for two round trips: 8 sequences at position 4,095, 8 kv
   // heads, 39.3 us with room for 8,192 positions, 28.3 with 4,096; now 31.2).
   static_assert(!LOOP || (NT && !RG && G > 1), "a loop needs the position first");
-  for (;; c += gridDim.x) {
+  for (;; c += a.cstep) {
   // (q again for each chunk: held over the loop it costs the second workgroup
   // of a CU its registers)
   if (LOOP) asm volatile("" ::: "memory");
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
     const int32_t pr = PG ? (a.lens ? a.lens[b] : a.pos[0]) : a.pos[0] + (a.qper ? (int32_t)(qr % a.qper) : 0);
     lim = (pr < 0 ? 0u : ((uint32_t)pr >= a.max_seq ? a.max_seq - 1 : (uint32_t)pr)) + 1;
     if (p0 >= lim) {  // block-uniform
-      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, gridDim.x);
+      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, a.cstep);
       else attn_no_chunk<HD, G>(a, pctx, pmz);
       return;
     }
@@ -427,7 +429,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
       pmz[2 * h + 1] = zz;
     }
   }
-  if (!LOOP || c + gridDim.x >= a.nchunk) return;
+  if (!LOOP || c + a.cstep >= a.nchunk) return;
   __syncthreads();  // the waves' partials have been read
   }
 }
@@ -496,7 +498,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
     return a.nsink + (t >= a.win ? t - a.win : t);
   };
   static_assert(!LOOP || (NT && !RG), "a loop needs the position first");
-  for (;; c += gridDim.x) {  // LOOP: as in k_attn_part
+  for (;; c += a.cstep) {  // LOOP: as in k_attn_part
   if (LOOP) asm volatile("" ::: "memory");
   const size_t cb = (size_t)qr * a.nchunk + c;
   float *pctx = a.pctx + cb * a.heads * HD + (size_t)h0 * HD;
@@ -521,7 +523,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
     lim = (pr < 0 ? 0u : ((uint32_t)pr >= a.max_seq ? a.max_seq - 1 : (uint32_t)pr)) + 1;
     len = lim;  // positions attended: 0 .. pr
     if (p0 >= lim) {  // block-uniform
-      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, gridDim.x);
+      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, a.cstep);
       else attn_no_chunk<HD, G>(a, pctx, pmz);
       return;
     }
@@ -752,7 +754,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       pmz[2 * h + 1] = zz;
     }
   }
-  if (!LOOP || c + gridDim.x >= a.nchunk) return;
+  if (!LOOP || c + a.cstep >= a.nchunk) return;
   __syncthreads();  // the waves' contexts have been read
   }
 }
@@ -907,16 +909,24 @@ static int attn_setup(AttnArgs &a, uint32_t batch, uint32_t heads, uint32_t kvhe
 // The chunk pass over `rows` query rows for a filled-in AttnArgs.  A
 // workgroup scores every query head of its kv head (K and V read once)
 // unless there are too few workgroups to spread over the CUs: then one head
-// each (K and V come from L2 for the others).
+// each (K and V come from L2 for the others).  A group of 8 heads takes two
+// workgroups of 4 on one XCD: the pass is bound by its VALU work, and the
+// registers of 8 heads' scores and contexts leave a CU one workgroup.  us, 8
+// heads a workgroup / 4 (4 kv heads): head_dim 128, 16 sequences at 4,000
+// 67 / 47, 64 at 2,000 109 / 86, 40 paged of up to 3,340 98 / 69; head_dim 64,
+// one at 16,000 19.7 / 14.2, 64 at 900 34 / 33.  (With the two on
+// different XCDs and looping over their chunks as below: 68 and 132, not 47 and 86.)
+// Ring caches and entry lists rotate each key per workgroup and stay at 8 (64
+// sequences over 2,048 entries, head_dim 128: 137 us, two of 4 169).
 static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int mode, hipStream_t st) {
   const uint32_t ni = attn_ni(head_dim, a.max_seq);
-  const uint32_t G = (uint64_t)rows * a.kvheads * a.nchunk >= 128 ? a.grp : 1;
+  const bool rot = mode == AM_RING || mode == AM_ENTRIES;
+  const uint32_t G = (uint64_t)rows * a.kvheads * a.nchunk >= 128 ? (rot ? a.grp : min(a.grp, 4u)) : 1;
   // positions attended per sequence at most: the cache (contiguous, ring) or
   // its block table's reach (paged); entry lists stay on plain loads
   const uint64_t seqs = a.qper ? (rows + a.qper - 1) / a.qper : rows;
   if (mode != AM_ENTRIES && seqs * a.kvheads * a.max_seq * head_dim * 4 >= ATTN_NT_BYTES) mode |= AM_NT;
   constexpr int AM_CONTIG_NT_ = AM_CONTIG | AM_NT;
-  a.nunits = rows * a.kvheads * a.nchunk;
   // Many chunks of a large cache: workgroups that loop over their unit's, four
   // per CU over contiguous caches (all at one position), eight over paged ones
   // (lengths differ, so they need more to balance).  us with 2 / 4 / 8 per CU:
@@ -927,18 +937,22 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
   const uint64_t units = (uint64_t)rows * (a.heads / G);
   const int bm0 = mode & 7;
   uint32_t gx = a.nchunk;
-  if (G > 1 && (mode & AM_NT) && (bm0 == AM_CONTIG || bm0 == AM_PAGED) && a.nchunk >= 8) {
+  if (G > 1 && G == a.grp && (mode & AM_NT) && (bm0 == AM_CONTIG || bm0 == AM_PAGED) && a.nchunk >= 8) {
     const uint64_t want = ((bm0 == AM_PAGED ? 8ull : 4ull) * nlg_num_cu() + units - 1) / units;
     if (want < gx) {
       gx = (uint32_t)want;
       mode |= AM_LOOP;
     }
   }
-  const dim3 grid = G == 1 ? dim3((a.nunits + 7) / 8 * 8 * a.grp) : dim3(gx, a.heads / G, rows);
+  a.cstep = gx;
+  // (a grid's x dimension holds fewer than 2^32 threads; past it the pair is in y)
+  const uint64_t nu = (uint64_t)rows * a.kvheads * gx;
+  a.nunits = (G == 1 || G < a.grp) && (nu + 7) * (a.grp / G) * (ATTN_WAVES * 64) < (1ull << 32) ? (uint32_t)nu : 0;
+  const dim3 grid = a.nunits ? dim3((a.nunits + 7) / 8 * 8 * (a.grp / G)) : dim3(gx, a.heads / G, rows);
   const dim3 blk(ATTN_WAVES * 64);
   // (ring caches small enough for plain loads keep the VALU pass: that
   // variant's registers spill under the two-workgroups-per-CU bound)
-  if (head_dim == 128 && G == 4 && ni == 8 &&
+  if (head_dim == 128 && a.grp == 4 && G == 4 && ni == 8 &&
       (bm0 == AM_CONTIG || mode == (AM_RING | AM_NT))) {
     const bool nt = mode & AM_NT, rg = bm0 == AM_RING;
     if (rg) {
@@ -957,22 +971,25 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
     else hipLaunchKernelGGL((k_attn_part<HD, GG, 4, PGV>), grid, blk, 0, st, a);           \
   } while (0)
 // (a loop: ni is 8 at 8 chunks and more, G at least 2)
+// (rows rotated by rank take 8 heads a workgroup, the others at most 4)
 #define AT(HD, GG)                                                                         \
   do {                                                                                     \
-    if (mode & AM_LOOP) {                                                                  \
-      if constexpr (GG > 1) {                                                              \
-        if (bm0 == AM_PAGED)                                                               \
-          hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_PAGED | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
-        else if constexpr (HD != 128 || GG != 4) /* those: matrix cores */                 \
-          hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_CONTIG | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
-      }                                                                                    \
-    } else if (mode == AM_PAGED) AT1(HD, GG, AM_PAGED);                                           \
-    else if (mode == (AM_PAGED | AM_NT)) AT1(HD, GG, AM_PAGED | AM_NT);                    \
-    else if (mode == AM_RING) AT1(HD, GG, AM_RING);                                        \
+    if (mode == AM_RING) AT1(HD, GG, AM_RING);                                             \
     else if (mode == (AM_RING | AM_NT)) AT1(HD, GG, AM_RING | AM_NT);                      \
     else if (mode == AM_ENTRIES) AT1(HD, GG, AM_ENTRIES);                                  \
-    else if (mode == AM_CONTIG_NT_) AT1(HD, GG, AM_CONTIG | AM_NT);                        \
-    else AT1(HD, GG, AM_CONTIG);                                                           \
+    else if constexpr (GG <= 4) {                                                          \
+      if (mode & AM_LOOP) {                                                                \
+        if constexpr (GG > 1) {                                                            \
+          if (bm0 == AM_PAGED)                                                             \
+            hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_PAGED | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
+          else if constexpr (HD != 128 || GG != 4) /* those: matrix cores */               \
+            hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_CONTIG | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
+        }                                                                                  \
+      } else if (mode == AM_PAGED) AT1(HD, GG, AM_PAGED);                                  \
+      else if (mode == (AM_PAGED | AM_NT)) AT1(HD, GG, AM_PAGED | AM_NT);                  \
+      else if (mode == AM_CONTIG_NT_) AT1(HD, GG, AM_CONTIG | AM_NT);                      \
+      else AT1(HD, GG, AM_CONTIG);                                                         \
+    }                                                                                      \
   } while (0)
   if (head_dim == 128) {
     if (G == 1) AT(128, 1); else if (G == 2) AT(128, 2); else if (G == 4) AT(128, 4); else AT(128, 8);
