@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecArgs a) {
 // context and (maximum, sum) for k_decode_merge; with 1 it writes C.
 // Bound by the K/V stream and, below a few MB, by the launches and the chain
 // position -> rows -> partials: 4 sequences of 2,048 positions, 20 heads over 5
-// of 128 (42 MB) 926 -> 22.4 us; one of 701 positions 240 -> 11.6; one of 8,001,
+// of 128 (42 MB) 926 -> 22.1 us; one of 701 positions 240 -> 11.6; one of 8,001,
 // 32 heads over 8 (66 MB) 3,680 -> 29.0 (2.3 TB/s); one of 32 9.5 -> 6.9.  k_decode_attn,
 // two passes of one position a wave at a time, stays for buffers that hold no
 // whole float4 rows.
@@ -153,8 +153,8 @@ __device__ __forceinline__ float lanes_sum(float v) {
   v = v + __int_as_float(nlg_dpp<0x4E>(__float_as_int(v)));   // quad_perm [2,3,0,1]
   v = v + __int_as_float(nlg_dpp<0x141>(__float_as_int(v)));  // row_half_mirror
   v = v + __int_as_float(nlg_dpp<0x140>(__float_as_int(v)));  // row_mirror
-  if (L >= 32) v = v + __shfl_xor(v, 16);
-  if (L >= 64) v = v + __shfl_xor(v, 32);
+  if (L >= 32) v = nlg_halve_f32<16>(v, v);
+  if (L >= 64) v = nlg_halve_f32<32>(v, v);
   return v;
 }
 

@@ -86,6 +86,28 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
+// Over the 64 / LPP lanes that hold the same dimensions, in every lane.
+// Exchanged on the VALU: through LDS, with four heads 16 exchanges of maxima and
+// sums and 64 of contexts a wave were a tenth of the pass (32 paged sequences of up
+// to 4,096 positions, 20 heads over 5 of 128: 53.2 -> 48.5 us).
+template <int LPP>
+__device__ __forceinline__ float part_max(float v) {
+  if (LPP == 8) {
+    const float o = __int_as_float(nlg_dpp<0x128>(__float_as_int(v)));  // row_ror:8
+    v = o > v ? o : v;
+  }
+  float2 r = nlg_pair_f32<16>(v);
+  v = r.y > r.x ? r.y : r.x;
+  r = nlg_pair_f32<32>(v);
+  return r.y > r.x ? r.y : r.x;
+}
+template <int LPP>
+__device__ __forceinline__ float part_sum(float v) {
+  if (LPP == 8) v = v + __int_as_float(nlg_dpp<0x128>(__float_as_int(v)));  // row_ror:8
+  v = nlg_halve_f32<16>(v, v);
+  return nlg_halve_f32<32>(v, v);
+}
+
 // Positions per workgroup for head dim HD: 8 waves x NI instructions x
 // (64 / (HD/8)) positions per instruction; NI = 8 when 4 would need more
 // chunks than the O-projection's prologue merges.
@@ -371,10 +393,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
     float mm = -1.0e30f;
 #pragma unroll
     for (int i = 0; i < NI; i++) mm = s[i][h] > mm ? s[i][h] : mm;
-    for (int off = LPP; off < 64; off <<= 1) {
-      const float o = __shfl_xor(mm, off);
-      mm = o > mm ? o : mm;
-    }
+    mm = part_max<LPP>(mm);
     m[h] = mm;
     z[h] = 0.0f;
 #pragma unroll
@@ -394,17 +413,25 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
       for (int j = 0; j < 8; j++) ctx[h][j] = fmaf(e, f16x8_at(vi, j), ctx[h][j]);
     }
   }
+  // The position groups' sums.  The G x 8 context values are halved at each of
+  // the last two steps: a lane ends with 2 G of them, from value v0 on.
+  float *cf = &ctx[0][0];
+  if (LPP == 8) {
+#pragma unroll
+    for (int v = 0; v < 8 * G; v++) cf[v] = cf[v] + __int_as_float(nlg_dpp<0x128>(__float_as_int(cf[v])));  // row_ror:8
+  }
+#pragma unroll
+  for (int v = 0; v < 4 * G; v++) cf[v] = nlg_halve_f32<16>(cf[v], cf[v + 4 * G]);
+#pragma unroll
+  for (int v = 0; v < 2 * G; v++) cf[v] = nlg_halve_f32<32>(cf[v], cf[v + 2 * G]);
+  const int v0 = (lane & 16 ? 4 * G : 0) + (lane & 32 ? 2 * G : 0);
+  if (LPP == 16 || !(lane & 8)) {
+#pragma unroll
+    for (int v = 0; v < 2 * G; v++) s_ctx[w][(v0 + v) / 8][d0 + (v0 + v) % 8] = cf[v];
+  }
 #pragma unroll
   for (int h = 0; h < G; h++) {
-    for (int off = LPP; off < 64; off <<= 1) {
-      z[h] = z[h] + __shfl_xor(z[h], off);
-#pragma unroll
-      for (int j = 0; j < 8; j++) ctx[h][j] = ctx[h][j] + __shfl_xor(ctx[h][j], off);
-    }
-    if (grp == 0) {
-#pragma unroll
-      for (int j = 0; j < 8; j++) s_ctx[w][h][d0 + j] = ctx[h][j];
-    }
+    z[h] = part_sum<LPP>(z[h]);
     if (lane == 0) {
       s_m[w][h] = m[h];
       s_z[w][h] = z[h];
@@ -676,12 +703,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       m = sc[bb][r] > m ? sc[bb][r] : m;
     }
   // the head's maximum over the wave: lanes li, li + 16, li + 32, li + 48
-  {
-    float o = __shfl_xor(m, 16);
-    m = o > m ? o : m;
-    o = __shfl_xor(m, 32);
-    m = o > m ? o : m;
-  }
+  m = part_max<16>(m);
   float z = 0.0f;
   v8h ph, pl;
 #pragma unroll
@@ -694,8 +716,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       ph[4 * bb + r] = h;
       pl[4 * bb + r] = (_Float16)(e - (float)h);
     }
-  z = z + __shfl_xor(z, 16);
-  z = z + __shfl_xor(z, 32);
+  z = part_sum<16>(z);
   // V^T tile: dims 8 li + e, slots 8 lg + 4 u + r (one wave's LDS operations
   // run in order, so the tile needs no barrier).  Rows past the position go
   // in as zeros: their probability is 0, but a cache row nobody wrote may

@@ -174,6 +174,25 @@ __device__ __forceinline__ float nlg_wave_max_f32(float v) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Lanes OFF (16 or 32) apart exchanged on the VALU instead of through LDS:
+// .x and .y are this lane's value and that of lane ^ OFF, in the lanes' order.
+template <int OFF>
+__device__ __forceinline__ float2 nlg_swap_f32(float a, float b) {
+  static_assert(OFF == 16 || OFF == 32, "rows of 16 lanes or halves of 32");
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  const auto r = OFF == 16 ? __builtin_amdgcn_permlane16_swap(x, y, false, false)
+                           : __builtin_amdgcn_permlane32_swap(x, y, false, false);
+  return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+template <int OFF>
+__device__ __forceinline__ float2 nlg_pair_f32(float v) { return nlg_swap_f32<OFF>(v, v); }
+// a + (a of lane ^ OFF) where lane & OFF is 0, the same of b in the others.
+template <int OFF>
+__device__ __forceinline__ float nlg_halve_f32(float a, float b) {
+  const float2 r = nlg_swap_f32<OFF>(a, b);
+  return r.x + r.y;
+}
+
 // Block-wide (blockDim.x multiple of 64, <= 1024) sum / max through LDS.
 // `scratch` needs blockDim.x/64 floats.  Every thread gets the result.
 // NW > 0 states the block's wave count at compile time (no read of the
