@@ -502,19 +502,46 @@ __global__ __launch_bounds__(256) void k_attn_gqa(GqaArgs a) {
 // makes the last query block seq / 32 key blocks long, and the longest
 // workgroup sets the time of a short prompt.  Bound by the matrix cores
 // (8,192 cycles a key block and wave at head dim 128): 20 heads over 5 of 128,
-// 1,024 positions 2,283 -> 82 us (65 TFLOP/s; 75 us with the loads taken out of
-// the loop, the rest is 2.5 rounds of workgroups), 4,096 positions 957 us (90
-// TFLOP/s of the 157 the f32 cores reach), 128 positions 10.6 us.  Four waves
+// 1,024 positions 2,283 -> 82 us (65 TFLOP/s of the 153 a large f32 product reaches;
+// 2.5 rounds of workgroups), 300 positions 22.5 us, 128 12.3, 16 9.8 (14.9 before).  Four waves
 // in two workgroups per CU measured the same; queries held in registers (one
 // wave per SIMD) 79 us at 1,024.
 // Keys past a query are masked in the scores; in the diagonal block their
 // probability of zero meets V rows the query does not attend, so there
 // infinities and NaNs of V are left out of the product and added for the
 // queries that attend them (0 x Inf would reach the others).
+// A score is summed in chains of 8 dimensions that meet in pairs.  One chain over
+// the head dimension rounds after each of them: 2-norm error against 64 bits at head
+// dim 128, 16 / 40 / 100 / 300 / 700 positions, the per-query kernel 0.89 / 1.13 /
+// 1.47 / 2.09 / 2.82e-7, one chain 1.62 / 2.13 / 2.52 / 2.90 / 3.15e-7, chains of 16
+// 0.88 / 1.10 / 1.27 / 1.42 / 1.57e-7, of 8 0.84 / 1.06 / 1.22 / 1.37 / 1.51e-7 at the same
+// time.  The pairs' sums need the registers that held the next block's K: a block
+// loads its own, and the other wave of the SIMD covers it (with both, 160 registers
+// spilled and 1,024 positions took 352 us, not 82).
 #define GQA_NW 8  // waves per workgroup
+typedef float gqa_v16f __attribute__((ext_vector_type(16)));
+template <int T0, int N>
+__device__ __forceinline__ gqa_v16f gqa_scores(const float4 *kv, const float *qp) {
+  gqa_v16f s;
+  if constexpr (N > 1) {
+    s = gqa_scores<T0, N / 2>(kv, qp);
+    s += gqa_scores<T0 + N / 2, N - N / 2>(kv, qp);
+  } else {
+#pragma unroll
+    for (int r = 0; r < 16; r++) s[r] = 0.0f;
+    const float4 q = *(const float4 *)(qp + 8 * T0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[T0].x, q.x, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[T0].y, q.y, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[T0].z, q.z, s, 0, 0, 0);
+    s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[T0].w, q.w, s, 0, 0, 0);
+  }
+  asm volatile("" : "+v"(s)::"memory");  // one chain after the other: K's registers free up as the sums need them
+  __builtin_amdgcn_sched_barrier(0);
+  return s;
+}
 template <int HD>
 __global__ __launch_bounds__(64 * GQA_NW) void k_gqa_mfma(GqaArgs a) {
-  typedef float v16f __attribute__((ext_vector_type(16)));
+  typedef gqa_v16f v16f;
   constexpr int KT = HD / 8, NT = (HD + 31) / 32, PITCH = 32 * NT + 4;
   __shared__ __align__(16) float s_o[GQA_NW][32][PITCH];
   __shared__ float s_m[GQA_NW][32], s_z[GQA_NW][32];
@@ -544,33 +571,27 @@ __global__ __launch_bounds__(64 * GQA_NW) void k_gqa_mfma(GqaArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; r++) o[n][r] = 0.0f;
   float m = NEG_BIG * NLG_LOG2E, z = 0.0f;  // z: this lane's half of the keys
-  if (qb >= (uint32_t)w) load_k(qb - w);
   __syncthreads();
   for (int64_t kb = (int64_t)qb - w; kb >= 0; kb -= GQA_NW) {
     const bool diag = kb == qb;
+    load_k((uint32_t)kb);
+    // V on its way before the scores, half of it once they have freed half of K's registers
     float v[16][NT];
+    auto load_v = [&](int t0, int t1) {
 #pragma unroll
-    for (int t = 0; t < 16; t++) {
-      const uint32_t key = (uint32_t)kb * 32 + (t % 4) + 8 * (t / 4) + 4 * g;
-      const float *vp = a.v.p + (size_t)(key < last ? key : last) * kvdim + kc;
+      for (int t = t0; t < t1; t++) {
+        const uint32_t key = (uint32_t)kb * 32 + (t % 4) + 8 * (t / 4) + 4 * g;
+        const float *vp = a.v.p + (size_t)(key < last ? key : last) * kvdim + kc;
 #pragma unroll
-      for (int n = 0; n < NT; n++) v[t][n] = vp[HD % 32 && 32 * n + i >= HD ? HD - 1 : 32 * n + i];
-    }
-    __builtin_amdgcn_sched_barrier(0);  // V on its way before the scores
-    asm volatile("" ::: "memory");      // the queries stay in LDS (not hoisted into registers)
-    v16f s;
-#pragma unroll
-    for (int r = 0; r < 16; r++) s[r] = 0.0f;
-#pragma unroll
-    for (int t = 0; t < KT; t++) {
-      const float4 q = *(const float4 *)&s_q[i][8 * t + 4 * g];
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[t].x, q.x, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[t].y, q.y, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[t].z, q.z, s, 0, 0, 0);
-      s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[t].w, q.w, s, 0, 0, 0);
-    }
-    if (kb >= GQA_NW) load_k((uint32_t)kb - GQA_NW);
-    __builtin_amdgcn_sched_barrier(0);  // the next K before this block's softmax
+        for (int n = 0; n < NT; n++) v[t][n] = vp[HD % 32 && 32 * n + i >= HD ? HD - 1 : 32 * n + i];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");  // the queries stay in LDS (not hoisted into registers)
+    };
+    load_v(0, 8);
+    v16f s = gqa_scores<0, KT / 2>(kv, &s_q[i][4 * g]);
+    load_v(8, 16);
+    s += gqa_scores<KT / 2, KT - KT / 2>(kv, &s_q[i][4 * g]);
     float bm = m;
 #pragma unroll
     for (int r = 0; r < 16; r++) {

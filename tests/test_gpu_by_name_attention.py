@@ -50,6 +50,29 @@ def test_prompt_attention_f32(seq, heads, kvh, hd):
     assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
 
 
+# 2-norm error against 64 bits.  A score rounded after each of 128 dimensions is
+# off by ~sqrt(128 / 2) half-ulps of its size, one summed in chains of 8 that meet
+# in pairs by ~sqrt(4 + 4); the first shows as 2.1e-7 of the result at 40
+# positions, the second as 1.06e-7, the rest (exponentials, sums) as 0.9e-7.
+@pytest.mark.parametrize("seq,hd,bar", [(40, 128, 1.5e-7), (40, 96, 1.5e-7), (300, 128, 2.1e-7)])
+def test_prompt_attention_f32_precision(seq, hd, bar):
+    heads, kvh = 8, 2
+    print(f"[gpu] attn-causal-gqa precision seq={seq} hd={hd}", flush=True)
+    q, k, v = inputs(seq, heads, kvh, hd)
+    q = (q / 1.5).astype(f32)
+    out = np.zeros(q.size, f32)
+    devs = [nlgpu.to_device(b) for b in (q, k, v, out)]
+    nlgpu.dispatch("attn-causal-gqa", devs, [seq, heads, kvh, hd], (heads * seq + 63) // 64)
+    got = devs[-1].download(f32, out.size).reshape(seq, heads, hd).astype(np.float64)
+    q64, k64, v64 = (b.astype(np.float64).reshape(seq, -1, hd) for b in (q, k, v))
+    s = np.einsum("qhd,khd->hqk", q64, np.repeat(k64, heads // kvh, axis=1)) / np.sqrt(hd)
+    s = np.where(np.tril(np.ones((seq, seq), bool)), s, -np.inf)
+    p = np.exp(s - s.max(axis=2, keepdims=True))
+    p /= p.sum(axis=2, keepdims=True)
+    want = np.einsum("hqk,khd->qhd", p, np.repeat(v64, heads // kvh, axis=1))
+    assert np.linalg.norm(got - want) <= bar * np.linalg.norm(want)
+
+
 @pytest.mark.parametrize("groups", [1, 3, 5])
 def test_prompt_attention_f32_partial_grid(groups):
     seq, heads, kvh, hd = 75, 6, 2, 64
