@@ -133,7 +133,7 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecArgs a) {
 // context and (maximum, sum) for k_decode_merge; with 1 it writes C.
 // Bound by the K/V stream and, below a few MB, by the launches and the chain
 // position -> rows -> partials: 4 sequences of 2,048 positions, 20 heads over 5
-// of 128 (42 MB) 926 -> 22.1 us; one of 701 positions 240 -> 11.6; one of 8,001,
+// of 128 (42 MB) 926 -> 22.0 us; one of 701 positions 240 -> 11.6; one of 8,001,
 // 32 heads over 8 (66 MB) 3,680 -> 29.0 (2.3 TB/s); one of 32 9.5 -> 6.9.  k_decode_attn,
 // two passes of one position a wave at a time, stays for buffers that hold no
 // whole float4 rows.
@@ -227,20 +227,23 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
         d = fmaf(q[h].w, k[i].w, d);
         if (!on) d = 0.0f;
         d = lanes_sum<L>(d);
-        s[i][h] = j0 + i * PPI + sub < jl ? d * coef : -INFINITY;
+        s[i][h] = j0 + i * PPI + sub < jl ? d : -INFINITY;
       }
 #pragma unroll
     for (int h = 0; h < G; h++) {
-      float bm = m[h];
+      // scaled once, in the exponent's FMA: a score rounded again by itself is off by
+      // half an ulp of the score, not of its distance to the maximum (2-norm error at 34
+      // positions, head dim 64: 1.31 -> 1.25e-7)
+      float bm = s[0][h] * coef > m[h] ? s[0][h] * coef : m[h];  // NaN never becomes the maximum
 #pragma unroll
-      for (int i = 0; i < DS_NI; i++) bm = s[i][h] > bm ? s[i][h] : bm;  // NaN never becomes the maximum
+      for (int i = 1; i < DS_NI; i++) bm = s[i][h] * coef > bm ? s[i][h] * coef : bm;
       const float al = nlg_exp2(m[h] - bm);
       m[h] = bm;
       z[h] *= al;
       cx[h].x *= al; cx[h].y *= al; cx[h].z *= al; cx[h].w *= al;
 #pragma unroll
       for (int i = 0; i < DS_NI; i++) {
-        const float e = nlg_exp2(s[i][h] - bm);
+        const float e = nlg_exp2(fmaf(s[i][h], coef, -bm));
         z[h] += e;
         cx[h].x = fmaf(e, v[i].x, cx[h].x);
         cx[h].y = fmaf(e, v[i].y, cx[h].y);
