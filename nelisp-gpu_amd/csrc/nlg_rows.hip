@@ -107,7 +107,6 @@ static int launch_softmax(const float *a, float *c, uint32_t rows, uint32_t n, h
   } while (0)
   if (n <= 64 * 4) SM(64, 4);
   else if (n <= SMW) SM(64, 16);
-  else if (n <= 256 * 4) SM(256, 4);
   else if (n <= 256 * 8) SM(256, 8);
   else if (n <= 256 * 16) SM(256, 16);
   else if (n <= 256 * 32) SM(256, 32);
