@@ -128,13 +128,17 @@ __global__ __launch_bounds__(256) void k_decode_attn(DecArgs a) {
 // eight waves walk blocks of DS_NI x PPI positions (float4 pieces, L lanes a
 // row, PPI = 64 / L rows an instruction) dealt round-robin over all waves of
 // all `nsplit` workgroups of the unit.  One pass: each block moves the wave's
-// running maximum, sum and context (scores in base 2), the next block's rows
-// already on their way.  With nsplit > 1 the workgroup leaves its partial
+// running maximum, sum and context, the next block's rows already on their way.
+// Maxima are kept as raw q.k and a difference is scaled where it is
+// exponentiated (dec_exp): it is exact near the maximum, so the largest element
+// weighs exactly 1 at any finite score (a maximum rounded after the scaling is off
+// by half its ulp, an exponent past 127 from scores of 1e10 on), and smaller
+// scores are rounded at their distance to the maximum.  With nsplit > 1 the workgroup leaves its partial
 // context and (maximum, sum) for k_decode_merge; with 1 it writes C.
 // Bound by the K/V stream and, below a few MB, by the launches and the chain
 // position -> rows -> partials: 4 sequences of 2,048 positions, 20 heads over 5
-// of 128 (42 MB) 926 -> 22.0 us; one of 701 positions 240 -> 11.6; one of 8,001,
-// 32 heads over 8 (66 MB) 3,680 -> 29.0 (2.3 TB/s); one of 32 9.5 -> 6.9.  k_decode_attn,
+// of 128 (42 MB) 927 -> 20.0 us; one of 701 positions 159 -> 9.4; one of 8,001,
+// 32 heads over 8 (66 MB) 3,794 -> 27.3 (2.4 TB/s); one of 32 9.4 -> 5.5.  k_decode_attn,
 // two passes of one position a wave at a time, stays for buffers that hold no
 // whole float4 rows.
 #define DS_WAVES 8
@@ -145,6 +149,9 @@ struct SplitArgs {
   uint32_t nsplit, hgroups;  // workgroups per (sequence, kv head, head group); head groups per kv head
   float *pctx, *pmz;         // [B][heads][nsplit][hd], [B][heads][nsplit][2]
 };
+
+// exp((s - m) / sqrt(hd)) of raw dot products, coef = log2(e) / sqrt(hd)
+__device__ __forceinline__ float dec_exp(float s, float m, float coef) { return nlg_exp2((s - m) * coef); }
 
 // Sum over aligned groups of L lanes (16, 32 or 64), in every lane.
 template <int L>
@@ -174,7 +181,7 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
   const uint64_t rows = base0 < a.ck.n ? (a.ck.n - base0) / a.kvdim : 0;
   const uint32_t jl = len < rows ? len : (uint32_t)rows;
   const bool on = 4u * dl < a.hd;
-  const float coef = NLG_LOG2E / sqrtf((float)a.hd);
+  const float coef = NLG_LOG2E / sqrtf((float)a.hd), least = NEG_BIG * sqrtf((float)a.hd);
   const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float4 q[G], cx[G];
   float m[G], z[G];
@@ -184,7 +191,7 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
     q[h] = *(const float4 *)(a.q.p + (size_t)bb * a.dim + (size_t)hh * a.hd + (on ? 4 * dl : 0));
     if (!on) q[h] = zero4;
     cx[h] = zero4;
-    m[h] = NEG_BIG * NLG_LOG2E;
+    m[h] = least;
     z[h] = 0.0f;
   }
   const size_t rb = base0 + kvh * a.hd + (on ? 4 * dl : 0);
@@ -231,19 +238,16 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
       }
 #pragma unroll
     for (int h = 0; h < G; h++) {
-      // scaled once, in the exponent's FMA: a score rounded again by itself is off by
-      // half an ulp of the score, not of its distance to the maximum (2-norm error at 34
-      // positions, head dim 64: 1.31 -> 1.25e-7)
-      float bm = s[0][h] * coef > m[h] ? s[0][h] * coef : m[h];  // NaN never becomes the maximum
+      float bm = s[0][h] > m[h] ? s[0][h] : m[h];  // NaN never becomes the maximum
 #pragma unroll
-      for (int i = 1; i < DS_NI; i++) bm = s[i][h] * coef > bm ? s[i][h] * coef : bm;
-      const float al = nlg_exp2(m[h] - bm);
+      for (int i = 1; i < DS_NI; i++) bm = s[i][h] > bm ? s[i][h] : bm;
+      const float al = dec_exp(m[h], bm, coef);
       m[h] = bm;
       z[h] *= al;
       cx[h].x *= al; cx[h].y *= al; cx[h].z *= al; cx[h].w *= al;
 #pragma unroll
       for (int i = 0; i < DS_NI; i++) {
-        const float e = nlg_exp2(fmaf(s[i][h], coef, -bm));
+        const float e = dec_exp(s[i][h], bm, coef);
         z[h] += e;
         cx[h].x = fmaf(e, v[i].x, cx[h].x);
         cx[h].y = fmaf(e, v[i].y, cx[h].y);
@@ -258,7 +262,7 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
 #pragma unroll
     for (int off = L; off < 64; off <<= 1) {
       const float om = __shfl_xor(m[h], off), mm = om > m[h] ? om : m[h];
-      const float al = nlg_exp2(m[h] - mm), ol = nlg_exp2(om - mm);
+      const float al = dec_exp(m[h], mm, coef), ol = dec_exp(om, mm, coef);
       z[h] = fmaf(z[h], al, __shfl_xor(z[h], off) * ol);
       cx[h].x = fmaf(cx[h].x, al, __shfl_xor(cx[h].x, off) * ol);
       cx[h].y = fmaf(cx[h].y, al, __shfl_xor(cx[h].y, off) * ol);
@@ -280,10 +284,10 @@ __global__ __launch_bounds__(64 * DS_WAVES) void k_decode_split(SplitArgs sa) {
     for (int k = 1; k < DS_WAVES; k++) mm = s_m[k][h] > mm ? s_m[k][h] : mm;
     const uint32_t out = split == 0 ? len - jl : 0u;  // positions past the caches: score 0, zero V
     if (out && 0.0f > mm) mm = 0.0f;
-    float zz = out ? (float)out * nlg_exp2(0.0f - mm) : 0.0f, c = 0.0f;
+    float zz = out ? (float)out * dec_exp(0.0f, mm, coef) : 0.0f, c = 0.0f;
 #pragma unroll
     for (int k = 0; k < DS_WAVES; k++) {
-      const float sc = nlg_exp2(s_m[k][h] - mm);
+      const float sc = dec_exp(s_m[k][h], mm, coef);
       zz = fmaf(s_z[k][h], sc, zz);
       c = fmaf(s_ctx[k][h][d], sc, c);
     }
@@ -309,8 +313,9 @@ __global__ __launch_bounds__(256) void k_decode_merge(SplitArgs sa) {
   if (threadIdx.x < 64) {
     const uint32_t t = threadIdx.x;
     const float *mz = sa.pmz + at * sa.nsplit * 2;
-    const float m = t < sa.nsplit ? mz[2 * t] : NEG_BIG * NLG_LOG2E, z = t < sa.nsplit ? mz[2 * t + 1] : 0.0f;
-    const float sc = nlg_exp2(m - nlg_wave_max_f32(m));
+    const float root = sqrtf((float)a.hd);
+    const float m = t < sa.nsplit ? mz[2 * t] : NEG_BIG * root, z = t < sa.nsplit ? mz[2 * t + 1] : 0.0f;
+    const float sc = dec_exp(m, nlg_wave_max_f32(m), NLG_LOG2E / root);
     s_w[t] = sc;
     const float zz = nlg_wave_sum_f32(z * sc);
     if (t == 0) s_z = zz;

@@ -231,6 +231,52 @@ def test_decode_attention_f32_infinities():
         assert np.max(np.abs(got[fine] - want[fine])) <= 1e-5 * np.max(np.abs(want[fine]))
 
 
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("size", [1e8, 1e10, 5e10, 1e15, 1e20])
+@pytest.mark.parametrize("heads,kvh,hd,maxseq,pos", [(4, 2, 128, 600, 0), (6, 2, 64, 300, 299), (8, 2, 128, 700, 511),
+                                                     (2, 2, 256, 200, 150)])
+def test_decode_attention_f32_large_scores(heads, kvh, hd, maxseq, pos, size, graph):
+    """q.k of any finite size.  Where every key is the same the values' mean is the
+    answer; where they differ by far more than 1 the largest score's value is."""
+    print(f"[gpu] decode-attn-b scores of {size:g} heads={heads}/{kvh} hd={hd} pos={pos} graph={graph}", flush=True)
+    q, k, v = decode_inputs(1, heads, kvh, hd, maxseq, seed=5)
+    push = [1, heads * hd, heads, kvh, maxseq]
+    val = v.reshape(maxseq, kvh, hd)[:pos + 1].astype(np.float64)
+    same = np.tile(k[:kvh * hd], maxseq).copy()
+    dots = np.einsum("hd,hd->h", q.reshape(heads, hd).astype(np.float64),
+                     np.repeat(same[:kvh * hd].reshape(kvh, hd), heads // kvh, axis=0))
+    qs = (q.reshape(heads, hd) * (size / np.abs(dots))[:, None]).astype(f32).reshape(-1)
+    got, _ = decode_both(qs, same, v, pos, push, graph=graph)
+    mean = np.repeat(val.mean(axis=0), heads // kvh, axis=0).reshape(-1)
+    assert np.max(np.abs(got - mean)) <= 1e-5 * np.max(np.abs(val))
+    got, _ = decode_both(qs, k, v, pos, push, graph=graph)
+    s = np.einsum("hd,jhd->jh", qs.reshape(heads, hd).astype(np.float64),
+                  np.repeat(k.reshape(maxseq, kvh, hd)[:pos + 1], heads // kvh, axis=1))
+    top = s.max(axis=0)
+    for h in range(heads):
+        near = s[:, h] >= top[h] - max(1e-4 * abs(top[h]), 1e3 * np.sqrt(hd))
+        if near.sum() == 1:  # an f32 score is good to ~1e-6 of itself
+            assert np.max(np.abs(got.reshape(heads, hd)[h] - val[int(s[:, h].argmax()), h // (heads // kvh)])) <= 1e-5
+
+
+# 2-norm error against 64 bits at 34 positions: the per-position kernel's own is 1.26e-7
+@pytest.mark.parametrize("hd", [64, 128])
+def test_decode_attention_f32_precision(hd):
+    batch, heads, kvh, maxseq, pos = 16, 20, 5, 60, 33
+    q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq, seed=9)
+    q = (q / 1.5).astype(f32)
+    got, _ = decode_both(q, k, v, pos, [batch, heads * hd, heads, kvh, maxseq])
+    q64 = q.astype(np.float64).reshape(batch, heads, hd)
+    k64, v64 = (np.repeat(x.astype(np.float64).reshape(batch, maxseq, kvh, hd)[:, :pos + 1], heads // kvh, axis=2)
+                for x in (k, v))
+    s = np.einsum("bhd,bjhd->bhj", q64, k64) / np.sqrt(hd)
+    p = np.exp(s - s.max(axis=2, keepdims=True))
+    want = np.einsum("bhj,bjhd->bhd", p / p.sum(axis=2, keepdims=True), v64).reshape(-1)
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print(f"[gpu] decode-attn-b error against 64 bits, head dim {hd}: {err:.3g}", flush=True)
+    assert err <= 1.3e-7
+
+
 def test_decode_attention_f32_general_form():
     """K shorter than V by part of a row: the general kernel (zeros past it)."""
     batch, heads, kvh, hd, maxseq, pos = 1, 4, 2, 64, 90, 89
