@@ -13,6 +13,7 @@
 // cache-relative positions.
 #include <math.h>
 
+#include "nlg_attn_grid.h"
 #include "nlg_internal.h"
 
 // fp16 element e (0..7) of eight packed in a uint4, as f32 (exact)
@@ -48,9 +49,7 @@ struct AttnArgs {
   // [0, trows) as zero rotations
   const int32_t *ent;
   uint32_t nslots, trows;
-  // workgroups of fewer than grp query heads (nunits not 0): units (row, kv
-  // head, first chunk) on a 1-D grid, a unit's grp / G workgroups on one XCD
-  uint32_t nunits;
+  uint32_t nunits;  // units on a 1-D grid, 0: a 3-D grid (attn_grid)
   uint32_t cstep;  // first chunks per (row, kv head): a looping workgroup's step
 };
 
@@ -111,7 +110,6 @@ __device__ __forceinline__ float part_sum(float v) {
 // Positions per workgroup for head dim HD: 8 waves x NI instructions x
 // (64 / (HD/8)) positions per instruction; NI = 8 when 4 would need more
 // chunks than the O-projection's prologue merges.
-#define ATTN_WAVES 8
 static inline uint32_t attn_ni(uint32_t hd, uint32_t max_seq) {
   const uint32_t cs4 = ATTN_WAVES * 4u * (64u / (hd / 8u));
   return (max_seq + cs4 - 1) / cs4 > NLG_ATTN_MAX_CHUNKS ? 8u : 4u;
@@ -182,21 +180,9 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // workgroup: chunk c, query heads h0 .. h0+G-1 (all of one kv head), query row qr
   uint32_t c, h0, qr;
-  if (G == 1 || (G == 4 && !LOOP && !RG && a.nunits)) {
-    // Workgroups are dealt to the 8 XCDs round-robin by id, and each XCD
-    // has its own L2: the n = grp / G workgroups of one (row, kv head, chunk)
-    // unit get ids u%8 + 8(q + n*(u/8)), all on XCD u%8, so the unit's K/V rows
-    // come from HBM once and from that L2 for the other heads.
-    const uint32_t n = a.grp / G;
-    const uint32_t id = blockIdx.x, rest = id >> 3, q = rest % n, u = (id & 7u) + 8u * (rest / n);
-    if (u >= a.nunits) return;
-    c = u % a.cstep;
-    const uint32_t r2 = u / a.cstep;
-    h0 = (r2 % a.kvheads) * a.grp + q * G;
-    qr = r2 / a.kvheads;
-  } else {
-    c = blockIdx.x; h0 = blockIdx.y * G; qr = blockIdx.z;
-  }
+  if (!attn_unit<G>(blockIdx.x, blockIdx.y, blockIdx.z, attn_reads_units(G, LOOP, RG) ? a.nunits : 0u, a.cstep,
+                    a.kvheads, a.grp, c, h0, qr))
+    return;
   const uint32_t kvh = h0 / a.grp;
   const uint32_t b = a.qper ? qr / a.qper : qr;                         // its sequence
   // AM_LOOP (large caches, whose position is in hand first): the workgroup takes
@@ -966,10 +952,9 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
     }
   }
   a.cstep = gx;
-  // (a grid's x dimension holds fewer than 2^32 threads; past it the pair is in y)
-  const uint64_t nu = (uint64_t)rows * a.kvheads * gx;
-  a.nunits = (G == 1 || G < a.grp) && (nu + 7) * (a.grp / G) * (ATTN_WAVES * 64) < (1ull << 32) ? (uint32_t)nu : 0;
-  const dim3 grid = a.nunits ? dim3((a.nunits + 7) / 8 * 8 * (a.grp / G)) : dim3(gx, a.heads / G, rows);
+  const AttnGrid ag = attn_grid(rows, a.kvheads, a.grp, G, gx);
+  a.nunits = ag.nunits;
+  const dim3 grid(ag.x, ag.y, ag.z);
   const dim3 blk(ATTN_WAVES * 64);
   // (ring caches small enough for plain loads keep the VALU pass: that
   // variant's registers spill under the two-workgroups-per-CU bound)

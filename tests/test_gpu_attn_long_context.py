@@ -97,3 +97,27 @@ def test_paged(heads, kvh, hd, bs, mbps):
     got = out.download(f32, q.size).reshape(q.shape)
     for b in range(batch):
         close(got[b], attend(q[b], *seqs[b]))
+
+
+@pytest.mark.parametrize("heads,kvh,batch", [(32, 32, 256), (64, 8, 512)])
+def test_paged_past_the_one_dimensional_grid(heads, kvh, batch):
+    """More chunk workgroups (2^23 of 512 threads) than a grid's x dimension holds,
+    one head each or two of a group's four."""
+    hd, bs, mbps = 64, 4096, 129  # 1,032 chunks of 512 positions; a pool that all sequences share
+    print(f"[gpu] paged attention heads={heads}/{kvh} batch={batch} reach={bs * mbps}", flush=True)
+    rng = np.random.default_rng(heads)
+    npool = 3
+    k, v = (rng.standard_normal((npool, bs, kvh, hd)).astype(np.float16) for _ in range(2))
+    q = rng.standard_normal((batch, heads, hd)).astype(f32)
+    lens = rng.integers(0, 1200, batch).astype(np.int32)
+    lens[[0, 100, batch - 1]] = [9000, 511, 4097]
+    table = rng.integers(0, npool, (batch, mbps)).astype(np.int32)
+    ws = nlgpu.DeviceArray(nlgpu.decode_attn_paged_f16_workspace(batch, heads, kvh, hd, bs, mbps))
+    dq, out = nlgpu.to_device(q), nlgpu.to_device(np.full(q.size, 7.0, f32))
+    nlgpu.decode_attn_paged_f16(dq, nlgpu.to_device(k), nlgpu.to_device(v), nlgpu.to_device(lens),
+                                nlgpu.to_device(table), npool, out, batch, heads, kvh, hd, bs, mbps, ws)
+    got = out.download(f32, q.size).reshape(q.shape)
+    for b in (0, 1, 100, batch // 2, batch - 1):
+        n = int(lens[b]) + 1
+        kk, vv = (x[table[b, :n // bs + 1]].reshape(-1, kvh, hd)[:n] for x in (k, v))
+        close(got[b], attend(q[b], kk, vv))
