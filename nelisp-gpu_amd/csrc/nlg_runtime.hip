@@ -88,8 +88,7 @@ int nlg_num_cu(void) { return g_num_cu; }
 
 hipStream_t nlg_stream(void *s) { return s ? (hipStream_t)s : g_stream; }
 
-// Library scratch for the batched linears' int8 activations, one per stream
-// (calls on different streams may run concurrently; calls on one stream run
+// Library scratch, one per stream and slot (calls on different streams may run concurrently; calls on one stream run
 // in order, so they can share).  Grown by allocating a larger buffer; older
 // ones stay allocated (a captured graph may still use them) until
 // nlg_shutdown.
@@ -102,7 +101,11 @@ static std::mutex g_scratch_mu;
 
 // Slot 0: the batched linears' int8 activations.  Slot 1: the column-split
 // GEMM's partial sums and arrival counters, zero-filled when allocated (the
-// GEMM leaves its counters at zero).
+// GEMM leaves its counters at zero).  Slot 2: the partials of the prompt
+// attention's key split.  Slot 3: those of decode-attn(-b), whose launch pairs
+// take a mutex of their own.
+// A refused allocation's error does not stay in the thread: a caller that goes
+// on without the scratch would find it at its launch check.
 static void *scratch_get(size_t bytes, hipStream_t st, int slot, bool quiet) {
   std::lock_guard<std::mutex> lk(g_scratch_mu);
   StreamScratch &e = g_scratch[{st, slot}];
@@ -118,11 +121,13 @@ static void *scratch_get(size_t bytes, hipStream_t st, int slot, bool quiet) {
   while (want < bytes) want *= 2;
   void *p = nullptr;
   if (hipMalloc(&p, want) != hipSuccess) {
+    (void)hipGetLastError();
     if (!quiet) nlg_fail("scratch: hipMalloc(%zu) failed", want);
     return nullptr;
   }
   if (slot == 1 && hipMemsetAsync(p, 0, want, st) != hipSuccess) {
     (void)hipFree(p);
+    (void)hipGetLastError();
     if (!quiet) nlg_fail("scratch: zero fill failed");
     return nullptr;
   }
