@@ -120,7 +120,13 @@ static void *scratch_get(size_t bytes, hipStream_t st, int slot, bool quiet) {
   size_t want = e.bytes ? e.bytes : (1u << 20);
   while (want < bytes) want *= 2;
   void *p = nullptr;
-  if (hipMalloc(&p, want) != hipSuccess) {
+  // the allocation is no part of a capture that runs on another stream (of this
+  // thread, or of any in the global mode) and must not end it
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  const hipError_t got = hipMalloc(&p, want);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  if (got != hipSuccess) {
     (void)hipGetLastError();
     if (!quiet) nlg_fail("scratch: hipMalloc(%zu) failed", want);
     return nullptr;

@@ -287,3 +287,32 @@ def test_decode_attention_f32_general_form():
     want = out.copy()
     orc.dispatch("decode-attn-b", [q.copy(), k[:k.size - 70].copy(), v.copy(), np.array([pos], f32), want], push, 4)
     assert np.max(np.abs(devs[-1].download(f32, out.size) - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+def test_decode_attention_f32_beside_a_capture():
+    """A call whose scratch is allocated while another stream of the thread is
+    being captured: it runs, and the capture stays valid."""
+    batch, heads, kvh, hd, maxseq, pos = 2, 4, 2, 64, 900, 800
+    q, k, v = decode_inputs(batch, heads, kvh, hd, maxseq)
+    push, groups = [batch, heads * hd, heads, kvh, maxseq], (batch * heads * hd + 63) // 64
+    x = np.arange(256, dtype=f32)
+    adds = [nlgpu.to_device(b) for b in (x, 2 * x, np.zeros(256, f32))]
+    devs = [nlgpu.to_device(b) for b in (q, k, v, np.array([pos], f32), np.zeros(batch * heads * hd, f32))]
+    captured, other = nlgpu.lib().nlg_stream_create(), nlgpu.lib().nlg_stream_create()
+    nlgpu.graph_begin(captured)
+    nlgpu.dispatch("vadd", adds, [256], 4, stream=captured)
+    rc = nlgpu.dispatch("decode-attn-b", devs, push, groups, stream=other, check=False)
+    nlgpu.dispatch("vadd", [adds[2], adds[0], adds[2]], [256], 4, stream=captured)
+    g = nlgpu.graph_end(captured)
+    assert rc == 0, nlgpu.last_error()
+    nlgpu.sync(other)
+    for _ in range(3):
+        nlgpu.graph_launch(g, captured)
+        nlgpu.sync(captured)
+        assert np.array_equal(adds[2].download(f32, 256), 4 * x)
+    nlgpu.graph_destroy(g)
+    want = np.zeros(batch * heads * hd, f32)
+    orc.dispatch("decode-attn-b", [q.copy(), k.copy(), v.copy(), np.array([pos], f32), want], push, groups)
+    assert np.max(np.abs(devs[-1].download(f32, want.size) - want)) <= 1e-5 * np.max(np.abs(want))
+    nlgpu.lib().nlg_stream_destroy(captured)
+    nlgpu.lib().nlg_stream_destroy(other)

@@ -1,7 +1,8 @@
 """The library's per-stream scratch (scratch_get, nelisp-gpu_amd/csrc/
 nlg_runtime.hip) against a stand-in for the few HIP calls that it makes, in a
 process of its own and without a GPU: an allocation that is refused leaves no
-error behind, which the next launch check would report as its own."""
+error behind, which the next launch check would report as its own, and one made
+while another stream is being captured asks for the relaxed mode."""
 import os
 import subprocess
 import sys
@@ -14,7 +15,10 @@ FAKE = r'''
 typedef int hipError_t;
 int refuse, last;                      /* the thread's last error */
 static hipError_t ret(int e) { if (e) last = e; return e; }
+int mode;                              /* of the thread: 0 global, 2 relaxed */
+hipError_t hipThreadExchangeStreamCaptureMode(int *m) { int o = mode; mode = *m; *m = o; return ret(0); }
 hipError_t hipMalloc(void **p, size_t n) {
+  if (mode != 2) return ret(900);      /* another stream is being captured */
   if (refuse) return ret(2);           /* hipErrorOutOfMemory */
   *p = malloc(n);
   return ret(0);
@@ -44,6 +48,7 @@ for slot in (1, 2, 3):
 refuse.value = 1
 assert get(5 << 20, 0x1000) is None and last.value == 0
 lib.nlg_last_error.restype = C.c_char_p
+assert C.c_int.in_dll(fake, "mode").value == 0  # given back
 assert b"hipMalloc" in lib.nlg_last_error()
 print("ok")
 '''
