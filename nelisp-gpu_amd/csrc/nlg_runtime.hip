@@ -108,7 +108,9 @@ static std::mutex g_scratch_mu;
 // on without the scratch would find it at its launch check.
 static void *scratch_get(size_t bytes, hipStream_t st, int slot, bool quiet) {
   std::lock_guard<std::mutex> lk(g_scratch_mu);
-  StreamScratch &e = g_scratch[{st, slot}];
+  // hipStreamPerThread's handle names another stream in every thread
+  static thread_local char own;
+  StreamScratch &e = g_scratch[{st == hipStreamPerThread ? (hipStream_t)&own : st, slot}];
   if (bytes <= e.bytes) return e.bufs.back();
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone) {

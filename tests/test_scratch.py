@@ -2,7 +2,8 @@
 nlg_runtime.hip) against a stand-in for the few HIP calls that it makes, in a
 process of its own and without a GPU: an allocation that is refused leaves no
 error behind, which the next launch check would report as its own, and one made
-while another stream is being captured asks for the relaxed mode."""
+while another stream is being captured asks for the relaxed mode; the per-thread
+stream's handle names another stream, and so another scratch, in every thread."""
 import os
 import subprocess
 import sys
@@ -45,6 +46,12 @@ for slot in (1, 2, 3):
     p = get_try(5 << 20, 0x1000, slot)
     assert p and get_try(1 << 20, 0x1000, slot) == p  # kept, per stream and slot
     assert get_try(1 << 20, 0x2000, slot) not in (None, p)
+import threading  # hipStreamPerThread (2) is another stream in every thread
+mine, other = get_try(1 << 20, 2, 3), []
+t = threading.Thread(target=lambda: other.extend(get_try(1 << 20, 2, 3) for _ in range(2)))
+t.start()
+t.join()
+assert mine and other[0] and other[0] == other[1] != mine == get_try(1 << 20, 2, 3)
 refuse.value = 1
 assert get(5 << 20, 0x1000) is None and last.value == 0
 lib.nlg_last_error.restype = C.c_char_p
