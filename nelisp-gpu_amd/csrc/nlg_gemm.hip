@@ -20,6 +20,7 @@
 // the reference's invocations gid < 64*groups (matmul-tiled: workgroups
 // wg < groups) would write; the rest of C is left as it was.
 #include "nlg_internal.h"
+#include "nlg_mm_tile.h"
 
 #define MM_T 16    // output tile edge
 #define MM_KC 256  // k per LDS stage
@@ -284,10 +285,15 @@ static void mmt_go(const float *A, const float *B, const float *bias, float *C, 
     hipLaunchKernelGGL((k_mmt<TM, TN, ORDER, true, true, VEC>), g, b, 0, st, A, B, bias, C, M, N, K, lim_mode, lim);
 }
 
+// whole float4s of A's and B's rows
+static bool mm_vec(const float *A, const float *B, uint32_t N, uint32_t K, bool trans_b) {
+  return K % 4 == 0 && (trans_b || N % 4 == 0) && (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
+}
+
 template <int TM, int TN>
 static void mmt(const float *A, const float *B, const float *bias, float *C, uint32_t M, uint32_t N, uint32_t K,
                 bool trans_b, int order, int lim_mode, uint64_t lim, hipStream_t st) {
-  const bool vec = K % 4 == 0 && (trans_b || N % 4 == 0) && (((uintptr_t)A | (uintptr_t)B) & 15) == 0;
+  const bool vec = mm_vec(A, B, N, K, trans_b);
   if (order == MM_TILE16) {
     if (vec) mmt_go<TM, TN, MM_TILE16, true>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
     else mmt_go<TM, TN, MM_TILE16, false>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
@@ -296,21 +302,16 @@ static void mmt(const float *A, const float *B, const float *bias, float *C, uin
     else mmt_go<TM, TN, MM_SERIAL, false>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
   }
 }
+
 static int mm(const float *A, const float *B, const float *bias, float *C, uint32_t M, uint32_t N, uint32_t K,
               bool trans_b, int order, int lim_mode, uint64_t lim, hipStream_t st, const char *name) {
   if (!M || !N || !lim) return NLG_OK;
   if (nlg_blocks(M, MM_T) > 65535) return nlg_fail("%s: M = %u is too large", name, M);
-  auto tiles = [&](uint64_t ta, uint64_t tb) { return ((M + ta - 1) / ta) * ((N + tb - 1) / tb); };
-  const uint64_t cu = nlg_num_cu();
-  // Larger tiles read less per product but need several workgroups per CU to
-  // issue at the full rate.  us with 64 x 64 / 64 x 32 / 32 x 32 / 16 x 16 tiles:
-  // 2,048^3 349 / 380 / 509 / 1,024; 1,536 x 1,024 x 1,536 (576 / 1,152 / 2,304
-  // tiles) 137 / 121 / 148 / 291; 1,024^3 81 / 56 / 71 / 133; 768^3 (144 / 288 /
-  // 576) 61 / 42 / 43 / 60; 512^3 42 / 26 / 16 / 20; 384^3 (36 / 72 / 144) 32 / 20 /
-  // 12.4 / 13.9; 64 x 2,048 x 2,048 (128 tiles of 32 x 32) 157 / 95 / 57 / 42.
-  if (K && tiles(64, 64) >= 3 * cu) mmt<4, 4>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
-  else if (K && tiles(64, 32) >= cu) mmt<4, 2>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
-  else if (K && tiles(32, 32) >= cu * 3 / 4) mmt<2, 2>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
+  const bool vec = mm_vec(A, B, N, K, trans_b);
+  const int form = K ? mm_tile(M, N, nlg_num_cu(), order == MM_TILE16, vec) : MM_16X16;
+  if (form == MM_64X64) mmt<4, 4>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
+  else if (form == MM_64X32) mmt<4, 2>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
+  else if (form == MM_32X32) mmt<2, 2>(A, B, bias, C, M, N, K, trans_b, order, lim_mode, lim, st);
   else if (order == MM_TILE16) mm_go<MM_TILE16>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
   else mm_go<MM_SERIAL>(A, B, bias, C, M, N, K, trans_b, lim_mode, lim, st);
   NLG_LAUNCHED(name);

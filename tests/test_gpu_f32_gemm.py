@@ -1,5 +1,5 @@
-"""The f32 products by name on their larger tiles (32, 64 and 128 outputs a
-side, chosen by how many of them fill the chip), bit for bit against the CPU
+"""The f32 products by name on their larger tiles (32 x 32, 64 x 32 and 64 x
+64 outputs, chosen by their estimated time: tests/test_mm_tile.py), bit for bit against the CPU
 restatement: ragged rows and columns, k at and around the LDS stages, aligned
 and unaligned row lengths, partial grids, -0 biases."""
 import numpy as np
@@ -40,7 +40,8 @@ def check(name, m, k, n, groups=None, seed=0):
 @pytest.mark.parametrize("name", ["matmul", "matmul-tiled", "linear"])
 @pytest.mark.parametrize("m,k,n", [(512, 32, 512), (530, 33, 515), (520, 1, 516), (16, 70, 9000),
                                    (1024, 40, 1024), (1030, 31, 1027), (40, 64, 20000),
-                                   (2048, 20, 2048), (2050, 17, 2041), (2052, 48, 2044)])
+                                   (2048, 20, 2048), (2050, 17, 2041), (2052, 48, 2044),
+                                   (2040, 17, 2035), (2036, 48, 2044), (33, 36, 8200), (1, 40, 32000)])
 def test_tiles_bit_exact(name, m, k, n):
     check(name, m, k, n)
 
