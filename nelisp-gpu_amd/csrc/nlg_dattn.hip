@@ -89,8 +89,21 @@ __device__ __forceinline__ float group_sum(float v) {
 // Exchanged on the VALU: through LDS, with four heads 16 exchanges of maxima and
 // sums and 64 of contexts a wave were a tenth of the pass (32 paged sequences of up
 // to 4,096 positions, 20 heads over 5 of 128: 53.2 -> 48.5 us).
-template <int LPP>
+// LDS: exchanged there all the same, in the same order (the same bits): the swaps'
+// pairs need registers, and the short ring forms of two and four heads lose the second
+// workgroup of a CU with them (head dim 64, four heads 114 -> 161 registers; 32
+// sequences over 1,024 slots, 32 heads over 8 23.1 us through LDS, 24.4 without; 16
+// over 8 19.3 / 20.9), the matrix-core ring form spills (2,048 slots, 20 heads over 5 of
+// 128: 46.8 / 48.3).  The other forms are up to 15% faster without LDS.
+template <int LPP, bool LDS = false>
 __device__ __forceinline__ float part_max(float v) {
+  if constexpr (LDS) {
+    for (int off = LPP; off < 64; off <<= 1) {
+      const float o = __shfl_xor(v, off);
+      v = o > v ? o : v;
+    }
+    return v;
+  }
   if (LPP == 8) {
     const float o = __int_as_float(nlg_dpp<0x128>(__float_as_int(v)));  // row_ror:8
     v = o > v ? o : v;
@@ -100,8 +113,12 @@ __device__ __forceinline__ float part_max(float v) {
   r = nlg_pair_f32<32>(v);
   return r.y > r.x ? r.y : r.x;
 }
-template <int LPP>
+template <int LPP, bool LDS = false>
 __device__ __forceinline__ float part_sum(float v) {
+  if constexpr (LDS) {
+    for (int off = LPP; off < 64; off <<= 1) v = v + __shfl_xor(v, off);
+    return v;
+  }
   if (LPP == 8) v = v + __int_as_float(nlg_dpp<0x128>(__float_as_int(v)));  // row_ror:8
   v = nlg_halve_f32<16>(v, v);
   return nlg_halve_f32<32>(v, v);
@@ -173,6 +190,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   constexpr bool NT = (MODE & AM_NT) != 0, LOOP = (MODE & AM_LOOP) != 0;
   constexpr bool PG = BM == AM_PAGED, RG = BM == AM_RING || BM == AM_ENTRIES, EN = BM == AM_ENTRIES;
   constexpr int LPP = HD / 8, PPI = 64 / LPP, PW = NI * PPI, NW = ATTN_WAVES, CS = NW * PW;
+  constexpr bool XL = BM == AM_RING && (NI == 4 ? G == 2 || G == 4 : HD == 128 && G == 4);  // see part_max
   __shared__ float s_m[NW][G], s_z[NW][G];
   __shared__ float s_ctx[NW][G][HD];
   asm volatile("" ::"s"(a.q), "s"(a.kc), "s"(a.vc), "s"(a.pos), "s"(a.pctx), "s"(a.pmz), "s"(a.heads),
@@ -379,7 +397,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
     float mm = -1.0e30f;
 #pragma unroll
     for (int i = 0; i < NI; i++) mm = s[i][h] > mm ? s[i][h] : mm;
-    mm = part_max<LPP>(mm);
+    mm = part_max<LPP, XL>(mm);
     m[h] = mm;
     z[h] = 0.0f;
 #pragma unroll
@@ -399,25 +417,42 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
       for (int j = 0; j < 8; j++) ctx[h][j] = fmaf(e, f16x8_at(vi, j), ctx[h][j]);
     }
   }
-  // The position groups' sums.  The G x 8 context values are halved at each of
-  // the last two steps: a lane ends with 2 G of them, from value v0 on.
-  float *cf = &ctx[0][0];
-  if (LPP == 8) {
+  // The position groups' sums.
+  if constexpr (XL) {
 #pragma unroll
-    for (int v = 0; v < 8 * G; v++) cf[v] = cf[v] + __int_as_float(nlg_dpp<0x128>(__float_as_int(cf[v])));  // row_ror:8
-  }
+    for (int h = 0; h < G; h++) {
+      for (int off = LPP; off < 64; off <<= 1) {
+        z[h] = z[h] + __shfl_xor(z[h], off);
 #pragma unroll
-  for (int v = 0; v < 4 * G; v++) cf[v] = nlg_halve_f32<16>(cf[v], cf[v + 4 * G]);
+        for (int j = 0; j < 8; j++) ctx[h][j] = ctx[h][j] + __shfl_xor(ctx[h][j], off);
+      }
+      if (grp == 0) {
 #pragma unroll
-  for (int v = 0; v < 2 * G; v++) cf[v] = nlg_halve_f32<32>(cf[v], cf[v + 2 * G]);
-  const int v0 = (lane & 16 ? 4 * G : 0) + (lane & 32 ? 2 * G : 0);
-  if (LPP == 16 || !(lane & 8)) {
+        for (int j = 0; j < 8; j++) s_ctx[w][h][d0 + j] = ctx[h][j];
+      }
+    }
+  } else {
+    // the G x 8 context values are halved at each of the last two steps: a lane
+    // ends with 2 G of them, from value v0 on
+    float *cf = &ctx[0][0];
+    if (LPP == 8) {
 #pragma unroll
-    for (int v = 0; v < 2 * G; v++) s_ctx[w][(v0 + v) / 8][d0 + (v0 + v) % 8] = cf[v];
+      for (int v = 0; v < 8 * G; v++) cf[v] = cf[v] + __int_as_float(nlg_dpp<0x128>(__float_as_int(cf[v])));  // row_ror:8
+    }
+#pragma unroll
+    for (int v = 0; v < 4 * G; v++) cf[v] = nlg_halve_f32<16>(cf[v], cf[v + 4 * G]);
+#pragma unroll
+    for (int v = 0; v < 2 * G; v++) cf[v] = nlg_halve_f32<32>(cf[v], cf[v + 2 * G]);
+    const int v0 = (lane & 16 ? 4 * G : 0) + (lane & 32 ? 2 * G : 0);
+    if (LPP == 16 || !(lane & 8)) {
+#pragma unroll
+      for (int v = 0; v < 2 * G; v++) s_ctx[w][(v0 + v) / 8][d0 + (v0 + v) % 8] = cf[v];
+    }
+#pragma unroll
+    for (int h = 0; h < G; h++) z[h] = part_sum<LPP>(z[h]);
   }
 #pragma unroll
   for (int h = 0; h < G; h++) {
-    z[h] = part_sum<LPP>(z[h]);
     if (lane == 0) {
       s_m[w][h] = m[h];
       s_z[w][h] = z[h];
@@ -689,7 +724,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       m = sc[bb][r] > m ? sc[bb][r] : m;
     }
   // the head's maximum over the wave: lanes li, li + 16, li + 32, li + 48
-  m = part_max<16>(m);
+  m = part_max<16, RG>(m);
   float z = 0.0f;
   v8h ph, pl;
 #pragma unroll
@@ -702,7 +737,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       ph[4 * bb + r] = h;
       pl[4 * bb + r] = (_Float16)(e - (float)h);
     }
-  z = part_sum<16>(z);
+  z = part_sum<16, RG>(z);
   // V^T tile: dims 8 li + e, slots 8 lg + 4 u + r (one wave's LDS operations
   // run in order, so the tile needs no barrier).  Rows past the position go
   // in as zeros: their probability is 0, but a cache row nobody wrote may
