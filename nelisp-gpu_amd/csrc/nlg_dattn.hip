@@ -49,7 +49,7 @@ struct AttnArgs {
   // [0, trows) as zero rotations
   const int32_t *ent;
   uint32_t nslots, trows;
-  uint32_t nunits;  // units on a 1-D grid, 0: a 3-D grid (attn_grid)
+  uint32_t nunits, clast;  // units on a 1-D grid, 0: a 3-D grid; its chunks last (attn_grid)
   uint32_t cstep;  // first chunks per (row, kv head): a looping workgroup's step
 };
 
@@ -198,17 +198,16 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   // workgroup: chunk c, query heads h0 .. h0+G-1 (all of one kv head), query row qr
   uint32_t c, h0, qr;
-  if (!attn_unit<G>(blockIdx.x, blockIdx.y, blockIdx.z, attn_reads_units(G, LOOP, RG) ? a.nunits : 0u, a.cstep,
-                    a.kvheads, a.grp, c, h0, qr))
+  if (!attn_unit<G>(blockIdx.x, blockIdx.y, blockIdx.z, attn_reads_units(G, LOOP, RG) ? a.nunits : 0u,
+                    BM == AM_CONTIG && NT ? a.clast : 0u, a.cstep, a.kvheads, a.grp, c, h0, qr))
     return;
   const uint32_t kvh = h0 / a.grp;
   const uint32_t b = a.qper ? qr / a.qper : qr;                         // its sequence
-  // AM_LOOP (large caches, whose position is in hand first): the workgroup takes
-  // chunks c, c + cstep, ... and stops at the first past the position,
-  // so room for a longer context costs no workgroups that find nothing to do
-  // (each holds a slot for two round trips: 8 sequences at position 4,095, 8 kv
-  // heads, 39.3 us with room for 8,192 positions, 28.3 with 4,096; now 31.2).
-  static_assert(!LOOP || (NT && !RG && G > 1), "a loop needs the position first");
+  // AM_LOOP (large paged caches, whose lengths are in hand first): the workgroup
+  // takes chunks c, c + cstep, ... and stops at the first past its length, so
+  // room for a longer context costs no workgroups that find nothing to do (each
+  // holds a slot for two round trips).
+  static_assert(!LOOP || (NT && PG && G > 1), "a loop needs the length first");
   for (;; c += a.cstep) {
   // (q again for each chunk: held over the loop it costs the second workgroup
   // of a CU its registers)
@@ -510,7 +509,7 @@ __global__ __launch_bounds__(512) void k_attn_part(AttnArgs a) {
 // reductions and conversions; here they are 32 matrix-core steps per wave.
 #define AMF_PITCH 36  // V^T tile row pitch in 16-bit elements (32 slots + 4: 8-byte aligned rows)
 
-template <bool NT, bool RG, bool LOOP = false>
+template <bool NT, bool RG>
 __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
   constexpr int HD = 128, G = 4, NW = ATTN_WAVES, PW = 32, CS = NW * PW;
   typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -522,10 +521,15 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
                "s"(a.kvheads), "s"(a.max_seq), "s"(a.nchunk), "s"(a.coef));
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, lg = lane >> 4;
-  uint32_t c = blockIdx.x;
-  const uint32_t h0 = blockIdx.y * G, qr = blockIdx.z;
+  uint32_t c, h0, qr;
+  (void)attn_unit<G>(blockIdx.x, blockIdx.y, blockIdx.z, 0u, NT && !RG ? a.clast : 0u, a.cstep, a.kvheads, a.grp, c, h0,
+                     qr);
   const uint32_t kvh = h0 / a.grp;
   const uint32_t b = a.qper ? qr / a.qper : qr;  // its sequence
+  const size_t cb = (size_t)qr * a.nchunk + c;
+  float *pctx = a.pctx + cb * a.heads * HD + (size_t)h0 * HD;
+  float *pmz = a.pmz + (cb * a.heads + h0) * 2;
+  const uint32_t p0 = c * CS, pw = p0 + w * PW;
   const size_t slot = (size_t)b * a.kvheads + kvh;
   const uint16_t *kb = a.kc + slot * a.max_seq * HD;
   const uint16_t *vb = a.vc + slot * a.max_seq * HD;
@@ -545,13 +549,6 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
     const uint32_t t = woff + (pc - a.nsink);  // < 2 win
     return a.nsink + (t >= a.win ? t - a.win : t);
   };
-  static_assert(!LOOP || (NT && !RG), "a loop needs the position first");
-  for (;; c += a.cstep) {  // LOOP: as in k_attn_part
-  if (LOOP) asm volatile("" ::: "memory");
-  const size_t cb = (size_t)qr * a.nchunk + c;
-  float *pctx = a.pctx + cb * a.heads * HD + (size_t)h0 * HD;
-  float *pmz = a.pmz + (cb * a.heads + h0) * 2;
-  const uint32_t p0 = c * CS, pw = p0 + w * PW;
   // q first (loads retire in issue order): lane (lg, li) takes head
   // h0 + li (li < 4; the others zero), dims 32 s + 8 lg .. + 7
   const float *qb = a.q + (size_t)qr * a.heads * HD + (size_t)(h0 + (li < G ? li : 0)) * HD + 8 * lg;
@@ -571,8 +568,7 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
     lim = (pr < 0 ? 0u : ((uint32_t)pr >= a.max_seq ? a.max_seq - 1 : (uint32_t)pr)) + 1;
     len = lim;  // positions attended: 0 .. pr
     if (p0 >= lim) {  // block-uniform
-      if (LOOP) attn_no_chunks<HD, G>(a, qr, h0, c, a.cstep);
-      else attn_no_chunk<HD, G>(a, pctx, pmz);
+      attn_no_chunk<HD, G>(a, pctx, pmz);
       return;
     }
   }
@@ -796,9 +792,6 @@ __global__ __launch_bounds__(512, 4) void k_attn_mfma(AttnArgs a) {
       pmz[2 * h + 1] = zz;
     }
   }
-  if (!LOOP || c + a.cstep >= a.nchunk) return;
-  __syncthreads();  // the waves' contexts have been read
-  }
 }
 
 // Pass 2: out = sum_c pctx_c * exp(m_c - M) / sum_c z_c * exp(m_c - M),
@@ -969,38 +962,45 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
   const uint64_t seqs = a.qper ? (rows + a.qper - 1) / a.qper : rows;
   if (mode != AM_ENTRIES && seqs * a.kvheads * a.max_seq * head_dim * 4 >= ATTN_NT_BYTES) mode |= AM_NT;
   constexpr int AM_CONTIG_NT_ = AM_CONTIG | AM_NT;
-  // Many chunks of a large cache: workgroups that loop over their unit's, four
-  // per CU over contiguous caches (all at one position), eight over paged ones
-  // (lengths differ, so they need more to balance).  us with 2 / 4 / 8 per CU:
-  // 8 sequences at 4,095 of 8,192, 8 kv heads 30.7 / 31.2 / 37.6 (39.3 one chunk
-  // each); 32 paged ones of up to 4,096, 5 kv heads 66 / 58 / 51.5 (60.7).  Of few
-  // chunks few are past the position and the loop only unbalances: 46 sequences,
-  // 8 kv heads, 5 chunks 38.4 / 40.8 / 36.3 (34.9).
+  // Many chunks of a large paged cache: workgroups that loop over their unit's, eight
+  // per CU (lengths differ, so they need more to balance).  us with 2 / 4 / 8 per
+  // CU: 32 sequences of up to 4,096, 5 kv heads 66 / 58 / 51.5 (60.7 one chunk each);
+  // where all lengths are equal the loop unbalances: 80 -> 83.
   const uint64_t units = (uint64_t)rows * (a.heads / G);
   const int bm0 = mode & 7;
   uint32_t gx = a.nchunk;
-  if (G > 1 && G == a.grp && (mode & AM_NT) && (bm0 == AM_CONTIG || bm0 == AM_PAGED) && a.nchunk >= 8) {
-    const uint64_t want = ((bm0 == AM_PAGED ? 8ull : 4ull) * nlg_num_cu() + units - 1) / units;
+  if (G > 1 && G == a.grp && mode == (AM_PAGED | AM_NT) && a.nchunk >= 8) {
+    const uint64_t want = (8ull * nlg_num_cu() + units - 1) / units;
     if (want < gx) {
       gx = (uint32_t)want;
       mode |= AM_LOOP;
     }
   }
   a.cstep = gx;
-  const AttnGrid ag = attn_grid(rows, a.kvheads, a.grp, G, gx);
-  a.nunits = ag.nunits;
-  const dim3 grid(ag.x, ag.y, ag.z);
-  const dim3 blk(ATTN_WAVES * 64);
+  // A large contiguous cache, all of it at one position: the chunks past the
+  // position start last, after every live one, instead of between them (each
+  // holds a slot for two round trips).  us, chunks first / last: 8 sequences at 4,095
+  // of 8,192, 32/8 heads of 128 39.2 / 31.7, of 64 24.7 / 17.4; 32 at 1,000 of 2,048,
+  // 20/5 heads of 128 28.6 / 21; full caches the same (16 of 2,300, 32/8 heads of 128
+  // 33 / 33; workgroups that loop over the chunks took 44.6), but for 64 sequences of
+  // 4,096, 32/8 heads of 128: 181 / 188.  Where the matrix-core form's workgroups are
+  // all resident at once the order only costs (8 of 2,048: 15.5 / 16.5).
   // (ring caches small enough for plain loads keep the VALU pass: that
   // variant's registers spill under the two-workgroups-per-CU bound)
-  if (head_dim == 128 && a.grp == 4 && G == 4 && ni == 8 &&
-      (bm0 == AM_CONTIG || mode == (AM_RING | AM_NT))) {
+  const bool mfma = head_dim == 128 && a.grp == 4 && G == 4 && ni == 8 &&
+                    (bm0 == AM_CONTIG || mode == (AM_RING | AM_NT));
+  const bool last = mode == (AM_CONTIG | AM_NT) && !(mfma && units * gx <= 2u * nlg_num_cu());
+  const AttnGrid ag = attn_grid(rows, a.kvheads, a.grp, G, gx, last);
+  a.nunits = ag.nunits;
+  a.clast = ag.clast;
+  const dim3 grid(ag.x, ag.y, ag.z);
+  const dim3 blk(ATTN_WAVES * 64);
+  if (mfma) {
     const bool nt = mode & AM_NT, rg = bm0 == AM_RING;
     if (rg) {
       hipLaunchKernelGGL((k_attn_mfma<true, true>), grid, blk, 0, st, a);
     } else {
-      if (mode & AM_LOOP) hipLaunchKernelGGL((k_attn_mfma<true, false, true>), grid, blk, 0, st, a);
-      else if (nt) hipLaunchKernelGGL((k_attn_mfma<true, false>), grid, blk, 0, st, a);
+      if (nt) hipLaunchKernelGGL((k_attn_mfma<true, false>), grid, blk, 0, st, a);
       else hipLaunchKernelGGL((k_attn_mfma<false, false>), grid, blk, 0, st, a);
     }
     NLG_LAUNCHED(rg ? "decode attention (ring fp16 KV, matrix cores)" : "decode attention (fp16 KV, matrix cores)");
@@ -1020,12 +1020,8 @@ static int attn_chunks_launch(AttnArgs &a, uint32_t rows, uint32_t head_dim, int
     else if (mode == AM_ENTRIES) AT1(HD, GG, AM_ENTRIES);                                  \
     else if constexpr (GG <= 4) {                                                          \
       if (mode & AM_LOOP) {                                                                \
-        if constexpr (GG > 1) {                                                            \
-          if (bm0 == AM_PAGED)                                                             \
-            hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_PAGED | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
-          else if constexpr (HD != 128 || GG != 4) /* those: matrix cores */               \
-            hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_CONTIG | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
-        }                                                                                  \
+        if constexpr (GG > 1)                                                              \
+          hipLaunchKernelGGL((k_attn_part<HD, GG, 8, AM_PAGED | AM_NT | AM_LOOP>), grid, blk, 0, st, a); \
       } else if (mode == AM_PAGED) AT1(HD, GG, AM_PAGED);                                  \
       else if (mode == (AM_PAGED | AM_NT)) AT1(HD, GG, AM_PAGED | AM_NT);                  \
       else if (mode == AM_CONTIG_NT_) AT1(HD, GG, AM_CONTIG | AM_NT);                      \

@@ -21,10 +21,13 @@ static int fail(const char *what, uint32_t rows, uint32_t kvh, uint32_t grp, int
 // one form: every workgroup (all: the whole grid; else a sample) reads a unit of
 // its own, and the grid is one that can be launched
 template <int G>
-int form(uint32_t rows, uint32_t kvh, uint32_t grp, uint32_t gx, bool loop, bool rot, bool all) {
-  const AttnGrid g = attn_grid(rows, kvh, grp, G, gx);
+int form(uint32_t rows, uint32_t kvh, uint32_t grp, uint32_t gx, bool loop, bool rot, bool all, bool last = false) {
+  if (!last && !loop && !rot && form<G>(rows, kvh, grp, gx, loop, rot, all, true)) return 1;  // chunks last too
+  const AttnGrid g = attn_grid(rows, kvh, grp, G, gx, last);
   if ((uint64_t)g.x * ATTN_WAVES * 64 >= (1ull << 32)) return fail("too many threads", rows, kvh, grp, G, gx);
   if (g.nunits && !attn_reads_units(G, loop, rot)) return fail("units not read", rows, kvh, grp, G, gx);
+  if (g.clast && (!last || g.nunits || g.z > 65535)) return fail("chunks last", rows, kvh, grp, G, gx);
+  uint32_t before = 0;
   const uint32_t nunits = attn_reads_units(G, loop, rot) ? g.nunits : 0u;
   const uint64_t want = (uint64_t)rows * kvh * (grp / G) * gx, total = (uint64_t)g.x * g.y * g.z;
   if (total < want) return fail("too few workgroups", rows, kvh, grp, G, gx);
@@ -33,7 +36,9 @@ int form(uint32_t rows, uint32_t kvh, uint32_t grp, uint32_t gx, bool loop, bool
   const uint64_t step = all ? 1 : total / 100003 + 1;
   for (uint64_t i = 0; i < total; i += step) {
     uint32_t c = ~0u, h0 = ~0u, qr = ~0u;
-    if (!attn_unit<G>(i % g.x, i / g.x % g.y, i / g.x / g.y, nunits, gx, kvh, grp, c, h0, qr)) continue;
+    if (!attn_unit<G>(i % g.x, i / g.x % g.y, i / g.x / g.y, nunits, g.clast, gx, kvh, grp, c, h0, qr)) continue;
+    if (g.clast && c < before) return fail("chunks not last", rows, kvh, grp, G, gx);
+    before = c;
     if (c >= gx || qr >= rows || h0 % G || h0 / G >= kvh * (grp / G) || h0 / grp != (h0 + G - 1) / grp)
       return fail("out of range", rows, kvh, grp, G, gx);
     const uint64_t at = ((uint64_t)qr * kvh * (grp / G) + h0 / G) * gx + c;
@@ -49,7 +54,8 @@ int main(void) {
   const struct { uint32_t rows, kvh, gx; bool all; } sizes[] = {
       {1, 1, 1, true}, {3, 5, 7, true}, {17, 3, 13, true}, {16, 8, 64, true}, {33, 1, 9, true},
       {255, 32, 1024, false}, {256, 32, 1023, false}, {256, 32, 1024, false}, {512, 32, 1024, false}, {65535, 8, 200, false},
-      {128, 32, 1024, false}, {129, 32, 1024, false}};
+      {128, 32, 1024, false}, {129, 32, 1024, false},
+      {2, 3, 65535, false}, {2, 3, 65536, false}};
   for (const auto &s : sizes)
     for (int rot = 0; rot < 2; rot++) {
       for (uint32_t grp = 1; grp <= 8; grp *= 2)

@@ -1,6 +1,6 @@
-"""fp16 decode attention over large caches of many chunks, where a workgroup
-takes several chunks of its unit and the merge skips those past the position:
-against float64, for the matrix-core and the vector form, contiguous and paged,
+"""fp16 decode attention over large caches of many chunks, where the chunks past
+the position start last (contiguous) or a workgroup takes several of its unit's
+(paged) and the merge skips those past the position: against float64, for the matrix-core and the vector form, contiguous and paged,
 at positions on and around the chunk edges; every row not attended holds NaN, and
 the workspace too (a chunk nobody wrote must not reach the result)."""
 import numpy as np
