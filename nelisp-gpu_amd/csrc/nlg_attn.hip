@@ -703,9 +703,7 @@ __global__ __launch_bounds__(64 * GQA_NW) void k_gqa_mfma(GqaArgs a) {
 
 // The matrix-core form reads whole float4 rows without bounds checks: every
 // buffer must hold its full extent, 16-byte aligned (V is read by elements),
-// and each kv head must serve the same number of query heads.  Taken at every
-// length: one query block already beats the per-query walk (2 x 128-lane
-// reductions per key) at 16 positions.
+// and each kv head must serve the same number of query heads.
 static bool gqa_mfma_ok(const GqaArgs &a) {
   const uint64_t rows = (uint64_t)a.heads * a.seq, qn = rows * a.hd, kn = (uint64_t)a.seq * a.kvheads * a.hd;
   const uintptr_t at = (uintptr_t)a.q.p | (uintptr_t)a.k.p | (uintptr_t)a.ctx;
@@ -730,21 +728,24 @@ int L_attn_causal_gqa(const nlg_buffer *b, const uint32_t *p, uint32_t groups, h
   a.ctx = (float *)b[3].ptr;
   a.nctx = b[3].nfloats;
   const dim3 blk(256);
-  if (gqa_mfma_ok(a)) {
-    const dim3 t((a.seq + 31) / 32 * a.heads);
-    bool took = true;
-    const dim3 blk(64 * GQA_NW);
-    if (a.hd == 128) hipLaunchKernelGGL(k_gqa_mfma<128>, t, blk, 0, st, a);
-    else if (a.hd == 96) hipLaunchKernelGGL(k_gqa_mfma<96>, t, blk, 0, st, a);
-    else if (a.hd == 80) hipLaunchKernelGGL(k_gqa_mfma<80>, t, blk, 0, st, a);
-    else if (a.hd == 64) hipLaunchKernelGGL(k_gqa_mfma<64>, t, blk, 0, st, a);
-    else if (a.hd == 32) hipLaunchKernelGGL(k_gqa_mfma<32>, t, blk, 0, st, a);
-    else took = false;
-    if (took) {
-      NLG_LAUNCHED("attn-causal-gqa");
-      return NLG_OK;
-    }
+  // A few queries: the walk over the keys (k_attn_gqa) is shorter than one key block
+  // of the matrix-core tile and the meeting of its waves.  us, walk / tile, 4 and 20
+  // heads alike: head dim 128, 1 / 4 / 8 / 9 queries 3.2 / 5.5 / 8.6 / 9.3 against 9.2-9.4;
+  // 96, 6 / 7 / 8: 7.1 / 7.8 / 8.7, 7.8; 80, 6 / 7: 7.1 / 7.8, 7.6; 64, 8 / 9: 6.1 / 6.5,
+  // 6.3; 32, 5 / 6: 4.6 / 5.0, 4.8.
+#define GQA_TILE(HD, WALK)                                                                \
+  if (a.hd == HD && a.seq > WALK && gqa_mfma_ok(a)) {                                     \
+    const dim3 t((a.seq + 31) / 32 * a.heads);                                            \
+    hipLaunchKernelGGL(k_gqa_mfma<HD>, t, dim3(64 * GQA_NW), 0, st, a);                   \
+    NLG_LAUNCHED("attn-causal-gqa");                                                      \
+    return NLG_OK;                                                                        \
   }
+  GQA_TILE(128, 8)
+  GQA_TILE(96, 7)
+  GQA_TILE(80, 6)
+  GQA_TILE(64, 8)
+  GQA_TILE(32, 5)
+#undef GQA_TILE
   const dim3 g(nlg_blocks(n, 4));
   if (a.hd <= 64) hipLaunchKernelGGL(k_attn_gqa<1>, g, blk, 0, st, a);
   else if (a.hd <= 128) hipLaunchKernelGGL(k_attn_gqa<2>, g, blk, 0, st, a);

@@ -50,6 +50,15 @@ def test_prompt_attention_f32(seq, heads, kvh, hd):
     assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 80, 96, 128])
+@pytest.mark.parametrize("seq", [2, 5, 6, 7, 8, 9])
+def test_prompt_attention_f32_few_queries(seq, hd):
+    """On both sides of the lengths up to which the walk over the keys is taken."""
+    q, k, v = inputs(seq, 6, 3, hd)
+    got, want = both(q, k, v, [seq, 6, 3, hd], (6 * seq + 63) // 64)
+    assert np.max(np.abs(got - want)) <= 1e-5 * np.max(np.abs(want))
+
+
 # 2-norm error against 64 bits.  A score rounded after each of 128 dimensions is
 # off by ~sqrt(128 / 2) half-ulps of its size, one summed in chains of 8 that meet
 # in pairs by ~sqrt(4 + 4); the first shows as 2.1e-7 of the result at 40
