@@ -922,9 +922,27 @@ __global__ __launch_bounds__(64 * NW) void k_ternary_mfma(TRowsArgs a) {
 
 // From this many tokens the matrix cores win: 6,912 x 2,560 at 2 / 4 / 8 tokens
 // 8.4 / 8.5 / 8.9 us against 7.3 / 11.2 / 21.2 with four tokens a wave, 2,560 x
-// 6,900 at 64 tokens 26 against 90.  The one loss is a few long rows: 1,000 x
-// 6,912 at 4 / 16 tokens 18.4 / 21.0 against 16.1 / 16.4.
+// 6,900 at 64 tokens 26 against 90.
 #define TROWS_MFMA 4
+
+// Few outputs: two rows and one token a wave (the same sums as the other forms of
+// k_ternary_rows, bit for bit), since a wave's chain over its row sets the time and
+// four rows or tokens make it longer.  us, one output a wave (x gathered) / four rows
+// a wave or the matrix cores / two rows a wave:
+//   aligned rows, 1-3 tokens: 1 x 512 x 512 3.5 / 3.4 / 2.8, 3 x 512 x 512 4.1 / 6.0 /
+//     2.8, 1 x 8,192 x 2,560 38 / 6.5 / 6.4, 2 x 6,912 x 2,560 72 / 7.8 / 8.9;
+//   more tokens: 4 x 256 x 14,336 28.7 / 34.0 / 11.1, 16 x 64 x 8,192 17.2 / 26.0 /
+//     7.2, 24 x 64 x 512 4.0 / 4.6 / 2.9; past that the matrix cores are within reach
+//     of it and their sums are the more accurate (4 x 512 x 512 4.1 / 4.0 / 2.8);
+//   other rows (x and w by elements: the vector unit's time is the tokens' times the
+//     rounds of waves): 1 x 512 x 2,562 7.2 / 8.4 / 7.2, 3 x 11.2 / 25.4 / 7.3, 8 x 20.0 /
+//     25.9 / 11.4; 1 x 2,560 x 2,562 15.9 / 8.6 / 11.2, 5 x 67 / 42.8 / 34.1.
+static bool trows_few(uint64_t srows, uint32_t out, bool xv, uint32_t t) {
+  const uint64_t cu = nlg_num_cu();
+  if (xv) return srows * out <= (srows >= TROWS_MFMA ? 6 : 32) * cu;
+  auto rounds = [&](uint64_t waves) { return (waves + 4 * cu - 1) / (4 * cu); };  // a wave per SIMD
+  return rounds((out + 1) / 2 * srows) <= t * rounds((uint64_t)((out + 3) / 4) * ((srows + t - 1) / t));
+}
 
 int L_ternary_rows(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipStream_t st) {
   const uint32_t seq = p[0], out = p[1], cols = p[2], nblk = p[3], wng = p[4];
@@ -941,7 +959,12 @@ int L_ternary_rows(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipS
               (float *)b[4].ptr, n, (uint32_t)srows, out, cols, nblk, wng, nw};
   const bool xv = cols % 4 == 0 && ((uintptr_t)a.x & 15) == 0 && cols;
   const dim3 blk(256);
-  if (xv && nw && srows >= TROWS_MFMA) {
+  const uint32_t t = srows >= 3 ? 4u : (uint32_t)srows;
+  if (trows_few(srows, out, xv, t)) {
+    const dim3 g((uint32_t)(srows * ((out + 7) / 8)));
+    if (xv) hipLaunchKernelGGL((k_ternary_rows<2, 1, true>), g, blk, 0, st, a);
+    else hipLaunchKernelGGL((k_ternary_rows<2, 1, false>), g, blk, 0, st, a);
+  } else if (xv && nw && srows >= TROWS_MFMA) {
     const bool wvec = wng % 4 == 0 && ((uintptr_t)a.wp & 15) == 0;
     // The smallest tiles that one round of workgroups covers, the largest past
     // that: 32- / 64-row tiles 10.2 / 13.4 us at 216 / 108 tiles, 25.9 / 17.1 at
@@ -956,7 +979,6 @@ int L_ternary_rows(const nlg_buffer *b, const uint32_t *p, uint32_t groups, hipS
     else if (wvec) hipLaunchKernelGGL((k_ternary_mfma<4, 4, true>), g, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((k_ternary_mfma<4, 4, false>), g, dim3(256), 0, st, a);
   } else {
-    const uint32_t t = srows >= 3 ? 4u : (uint32_t)srows;
     const dim3 g((uint32_t)((srows + t - 1) / t * ((out + 15) / 16)));
     if (xv) {
       if (t == 4) hipLaunchKernelGGL((k_ternary_rows<4, 4, true>), g, blk, 0, st, a);

@@ -1,5 +1,5 @@
-"""ternary-rows by name (f32 activations) on its two forms, a few rows and
-tokens per wave and 32-token tiles on the bf16 matrix cores, against the CPU
+"""ternary-rows by name (f32 activations) on its forms, two or four rows and
+up to four tokens per wave and 32-token tiles on the bf16 matrix cores, against the CPU
 restatement: edges of the tiles and of the 128-column blocks, word strides and
 block counts that cover more or less than the columns, partial grids,
 infinities and NaNs, buffers that are not 16-byte aligned."""
@@ -68,6 +68,15 @@ def test_ternary_rows(seq, out, cols, nblk, wng):
 @pytest.mark.parametrize("seq,out,cols", [(200, 9400, 132), (130, 2500, 1300), (33, 8200, 132)])
 def test_ternary_rows_many_tiles(seq, out, cols):
     """Enough tiles for 64- and 128-row workgroups."""
+    nblk, wng = (cols + 127) // 128, (cols + 15) // 16
+    got, want = both(*inputs(seq, out, cols, nblk, wng), [seq, out, cols, nblk, wng])
+    close(got, want, cols)
+
+
+@pytest.mark.parametrize("seq,out,cols", [(1, 8300, 256), (2, 4200, 256), (3, 2800, 256), (1, 2600, 37), (2, 2600, 37),
+                                          (4, 2600, 37), (5, 2700, 302), (24, 64, 512), (25, 64, 512)])
+def test_ternary_rows_many_outputs(seq, out, cols):
+    """Few tokens past the counts of outputs up to which a wave takes two rows."""
     nblk, wng = (cols + 127) // 128, (cols + 15) // 16
     got, want = both(*inputs(seq, out, cols, nblk, wng), [seq, out, cols, nblk, wng])
     close(got, want, cols)
