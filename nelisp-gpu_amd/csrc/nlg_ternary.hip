@@ -771,8 +771,8 @@ __global__ __launch_bounds__(256) void k_ternary_rows(TRowsArgs a) {
 // waves every NW-th 128-column block.
 //  * The weights {-2, -1, 0, 1} are exact in bf16 (byte permutes out of two
 //    four-entry tables).  An activation is split by truncation into three bf16
-//    values of 8 significant bits each, x = hi + mid + lo exactly, so every
-//    product is exact and the sums are f32 as before; hi has its own
+//    values of 8 significant bits each, x = hi + mid + lo exactly (from 2^-109 up:
+//    below), so every product is exact and the sums are f32 as before; hi has its own
 //    accumulator, so the small parts' additions round at their own size (all
 //    in one: error against 64 bits 1.2e-07, apart 6.8e-08, before 1.0e-07).
 //  * Step t of a block contracts word t of each row: lane half g takes fields
@@ -782,7 +782,11 @@ __global__ __launch_bounds__(256) void k_ternary_rows(TRowsArgs a) {
 //  * Per block the sum is scaled by the row's beta and added to the wave's total
 //    in LDS (registers hold no more), where the waves' totals then meet.
 // An infinity's remainders are NaN, so every output that sees one is NaN: such
-// outputs are summed again, one by one, in plain f32.
+// outputs are summed again, one by one, in plain f32.  So are those that the bits
+// below 2^-133, bf16's smallest, could show in: an activation below 2^-109 loses less
+// than 2^-132 a product, which shows in outputs of no more than 2^26 times that.
+// They are looked for at the end, among the outputs that small (a check of every
+// activation as it is split cost 4-20%): a zero one has its token's row read again.
 // Bound by the vector unit (the split of x, 44 instructions a step, and the
 // decode of the weights, 14 a row block, against 96 matrix-core cycles a row
 // block).  6,912 x 2,560: 64 tokens 1,929 -> 17.1 us (133 TFLOP/s), 16 tokens
@@ -898,25 +902,55 @@ __global__ __launch_bounds__(64 * NW) void k_ternary_mfma(TRowsArgs a) {
       for (int r = 0; r < 16; r++) tot(n, r) = fmaf(be[n], hi[n][r] + lo[n][r], tot(n, r));
   }
   __syncthreads();
+  auto merged = [&](uint32_t t, uint32_t n, uint32_t j) {
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NW; k++) v += s_c[k][n][t][j];
+    return v;
+  };
+  auto plain = [&](uint32_t s, uint32_t o) {
+    float v = 0.0f;
+    for (uint32_t b = 0; b < nb; b++) {
+      float part = 0.0f;
+      for (uint32_t c = 128 * b; c < 128 * b + 128 && c < keff; c++) {
+        const uint32_t w = a.wp[(size_t)o * a.wng + c / 16];
+        part += (float)((int32_t)(w << (30 - 2 * (c % 16))) >> 30) * a.x[(size_t)s * a.cols + c];
+      }
+      v += a.beta[(size_t)o * a.nblk + b] * part;
+    }
+    return v;
+  };
+  bool low = false;
   for (uint32_t e = threadIdx.x; e < 32 * 32 * RB; e += 64 * NW) {
     const uint32_t t = e / (32 * RB), n = e / 32 % RB, j = e % 32, s = s0 + t, o = o0 + 32 * n + j;
     const uint64_t idx = (uint64_t)s * a.out + o;
     if (s >= a.seq || o >= a.out || idx >= a.n) continue;
-    float v = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NW; k++) v += s_c[k][n][t][j];
-    if (v != v) {
-      v = 0.0f;
-      for (uint32_t b = 0; b < nb; b++) {
-        float part = 0.0f;
-        for (uint32_t c = 128 * b; c < 128 * b + 128 && c < keff; c++) {
-          const uint32_t w = a.wp[(size_t)o * a.wng + c / 16];
-          part += (float)((int32_t)(w << (30 - 2 * (c % 16))) >> 30) * a.x[(size_t)s * a.cols + c];
-        }
-        v += a.beta[(size_t)o * a.nblk + b] * part;
-      }
-    }
+    float v = merged(t, n, j);
+    low = low || fabsf(v) < 0x1p-20f;
+    if (v != v) v = plain(s, o);
     a.y[idx] = __fadd_rn(a.bias[o], v);
+  }
+  if (!__any(low)) return;
+  for (uint32_t e = threadIdx.x; e < 32 * 32 * RB; e += 64 * NW) {
+    const uint32_t t = e / (32 * RB), n = e / 32 % RB, j = e % 32, s = s0 + t, o = o0 + 32 * n + j;
+    const uint64_t idx = (uint64_t)s * a.out + o;
+    bool small = s < a.seq && o < a.out && idx < a.n && fabsf(merged(t, n, j)) < 0x1p-20f;
+    if (small) {  // 2^26 x (128 columns x 2^-132) x sum |BETA|: below 2^-20 for sums up to 2^79
+      float sum = 0.0f;
+      for (uint32_t b = 0; b < nb; b++) sum += fabsf(a.beta[(size_t)o * a.nblk + b]);
+      small = fabsf(merged(t, n, j)) <= sum * 0x1p-99f;
+    }
+    for (uint64_t todo = __ballot(small); todo;) {  // one of the wave's tokens at a time
+      const uint32_t tt = __builtin_amdgcn_readlane(t, __ffsll((unsigned long long)todo) - 1);
+      bool cut = false;
+      for (uint32_t c = lane; c < keff; c += 64) {
+        const float x = fabsf(a.x[(size_t)(s0 + tt) * a.cols + c]);
+        cut = cut || (x < 0x1p-109f && x != 0.0f);
+      }
+      const bool mine = small && t == tt;
+      if (__any(cut) && mine) a.y[idx] = __fadd_rn(a.bias[o], plain(s, o));
+      todo &= ~__ballot(mine);
+    }
   }
 }
 

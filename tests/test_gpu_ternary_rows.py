@@ -115,3 +115,23 @@ def test_ternary_rows_non_finite_and_wide(seq):
     assert np.isinf(want[1]).any() and np.isnan(want[1]).any() and np.isnan(want[2]).all()
     close(got[:3].reshape(-1), want[:3].reshape(-1), cols)
     close(got[3], want[3], cols)
+
+
+@pytest.mark.parametrize("seq,out", [(3, 70), (40, 70), (70, 300)])
+def test_ternary_rows_tiny_activations(seq, out):
+    """Rows of activations near and below the smallest normal number, whose lower
+    parts no bf16 holds, each compared on its own scale (beta 1, no bias)."""
+    cols, nblk, wng = 260, 3, 17
+    push = [seq, out, cols, nblk, wng]
+    x, w, bias, beta = inputs(seq, out, cols, nblk, wng)
+    x = x.reshape(seq, cols)
+    exps = [0, -90, -100, -108, -112, -115, -120, -126, -132, -140, -147]
+    for r in range(seq):
+        x[r] = np.ldexp(x[r].astype(np.float64), exps[r % len(exps)]).astype(f32)
+    x[0, ::2] = np.ldexp(1.5, -130)  # among normal ones
+    got, want = both(x.reshape(-1), w, 0 * bias, np.ones_like(beta), push)
+    got, want = got.reshape(seq, out), want.reshape(seq, out)
+    bar = min(1e-5, 8 * np.sqrt(cols) * 2.0 ** -24)
+    for r in range(seq):
+        err = np.max(np.abs(got[r].astype(np.float64) - want[r]))
+        assert err <= bar * np.max(np.abs(want[r])) + cols * 2.0 ** -149, (r, exps[r % len(exps)], err, np.max(np.abs(want[r])))
