@@ -378,13 +378,13 @@ int rows_t(const nlg_buffer *b, uint32_t out, uint32_t cols, uint32_t nblk, uint
   a.wcols = two_bit ? (cols + 15) / 16 : (cols + 3) / 4;
   const uint32_t seqs = (uint32_t)((dom + cols - 1) / cols);
   a.seq = seqs < seq ? seqs : seq;  // positions with an element in the domain
+  if (a.seq > 65535) return nlg_fail("%s: %u positions > 65535", k, a.seq);
   if (two_bit && rows_t_mfma(a, st)) {
     NLG_LAUNCHED(k);
     return NLG_OK;
   }
   const uint32_t cg = two_bit ? 64u : 32u;
   const dim3 grid((cols + cg - 1) / cg, a.seq), blk(256);
-  if (a.seq > 65535) return nlg_fail("%s: %u positions > 65535", k, a.seq);
   if (two_bit) hipLaunchKernelGGL(k_rows_t<16>, grid, blk, 0, st, a);
   else hipLaunchKernelGGL(k_rows_t<4>, grid, blk, 0, st, a);
   NLG_LAUNCHED(k);

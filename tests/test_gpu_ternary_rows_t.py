@@ -73,6 +73,15 @@ def test_ternary_rows_t_forms(seq, cols):
     assert same(got, want) and (want == -7.0).any()
 
 
+def test_ternary_rows_t_too_many_positions():
+    """More than 65,535 positions are refused, whichever form would take them."""
+    w, beta, g, push = inputs(3, 16, 1, 65536)
+    devs = [nlgpu.to_device(b) for b in (w, beta, g, np.full(16 * 65536, -7.0, f32))]
+    with pytest.raises(nlgpu.NlgError, match="65535"):
+        nlgpu.dispatch("ternary-rows-t", devs, push, 65536 * 16 // 64)
+    assert np.all(devs[3].download(f32, 1024) == -7.0)
+
+
 @pytest.mark.parametrize("seq,cols", [(2, 17000), (2, 200), (24, 2000), (66, 1300), (260, 20000)])
 def test_ternary_rows_t_extremes(seq, cols):
     """Products and sums below the normal range; infinities and NaNs of G; and
