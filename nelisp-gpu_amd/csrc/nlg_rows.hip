@@ -1,15 +1,18 @@
 // nlg_rows.hip -- row reductions: softmax, RMSNorm (istd, per-head).
 //
 // The reference gives each row to one invocation, which walks it serially
-// three times (softmax, kernels.el:28-42).  Here a workgroup owns a row: the
-// row is read from HBM once into registers (16 floats per thread at 4096
-// columns, non-temporal float4 loads), reduced with DPP within waves and LDS
-// across them, and written once (non-temporal stores) -- 8 bytes of traffic
-// per element, the minimum for an in-place softmax.  Reduction order differs from the serial reference, so
-// parity is by tolerance (<= 1e-5 relative for softmax, 1e-4 for RMSNorm).
+// three times (softmax, kernels.el:28-42).  Here a wave or a workgroup owns a
+// row (softmax_threads): it is read from HBM once into registers (16 floats per
+// thread at 4096 columns, non-temporal float4 loads), reduced with DPP within
+// waves and LDS across them, and written once (non-temporal stores) -- 8 bytes of
+// traffic per element, the minimum for an in-place softmax; only rows of more than
+// 32,768 columns are read three times.  Reduction order differs from the serial
+// reference, so parity is by tolerance (<= 1e-5 relative for softmax, 1e-4 for
+// RMSNorm).
 #include <math.h>
 
 #include "nlg_internal.h"
+#include "nlg_softmax_form.h"
 
 #define EPS6 0.000001f
 
@@ -94,25 +97,30 @@ __global__ __launch_bounds__(256) void k_softmax_stream(const float *a, float *c
   for (uint32_t i = threadIdx.x; i < n; i += 256) cr[i] = expf(__fsub_rn(ar[i], mx)) / s;
 }
 
-#define SMW 1024
-
 static int launch_softmax(const float *a, float *c, uint32_t rows, uint32_t n, hipStream_t st) {
   if (!rows || !n) return NLG_OK;
   const bool v4 = (n % 4 == 0) && ((((uintptr_t)a) | ((uintptr_t)c)) & 15) == 0;
+  const uint32_t tpr = softmax_threads(rows, n, v4, nlg_num_cu());
 #define SM(TPR, EPT)                                                                                   \
   do {                                                                                                 \
-    const dim3 g(TPR == 64 ? (rows + 3) / 4 : rows), b(TPR == 64 ? 256 : TPR);                         \
+    const dim3 g(TPR == 64 ? (uint32_t)(((uint64_t)rows + 3) / 4) : rows), b(TPR == 64 ? 256 : TPR);   \
     if (v4) hipLaunchKernelGGL((k_softmax_reg<TPR, EPT, true>), g, b, 0, st, a, c, rows, n);           \
     else hipLaunchKernelGGL((k_softmax_reg<TPR, EPT, false>), g, b, 0, st, a, c, rows, n);             \
   } while (0)
-  if (n <= 64 * 4) SM(64, 4);
-  else if (n <= SMW) SM(64, 16);
-  else if (n <= 256 * 8) SM(256, 8);
-  else if (n <= 256 * 16) SM(256, 16);
-  else if (n <= 256 * 32) SM(256, 32);
-  else if (n <= 1024 * 16) SM(1024, 16);
-  else if (n <= 1024 * 32) SM(1024, 32);
-  else hipLaunchKernelGGL(k_softmax_stream, dim3(rows), dim3(256), 0, st, a, c, rows, n);
+  if (tpr == 64) {
+    if (n <= 64 * 4) SM(64, 4);
+    else SM(64, 16);
+  } else if (tpr == 256) {
+    if (n <= 256 * 4) SM(256, 4);
+    else if (n <= 256 * 8) SM(256, 8);
+    else if (n <= 256 * 16) SM(256, 16);
+    else SM(256, 32);
+  } else if (tpr == 1024) {
+    if (n <= 1024 * 16) SM(1024, 16);
+    else SM(1024, 32);
+  } else {
+    hipLaunchKernelGGL(k_softmax_stream, dim3(rows), dim3(256), 0, st, a, c, rows, n);
+  }
 #undef SM
   NLG_LAUNCHED("softmax");
   return NLG_OK;

@@ -83,3 +83,17 @@ def test_softmax_row_widths(n, inplace):
     e = np.exp(x[live] - x[live].max(axis=1, keepdims=True))
     exact = e / e.sum(axis=1, keepdims=True)
     assert np.max(np.abs(got[live] - exact) / exact) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,n", [(1025, 257), (1030, 511), (513, 512), (1029, 777), (9, 1000), (1027, 1021), (515, 1024)])
+def test_softmax_many_rows(rows, n):
+    """257 to 1,024 columns in a wave each, past the rows that 256 threads take."""
+    print(f"[gpu] softmax rows={rows} n={n}", flush=True)
+    a = nlgpu.normal(n, rows * n, 3.0).reshape(rows, n)
+    a[3, n // 2:] = -np.inf
+    dc = nlgpu.DeviceArray(a.nbytes)
+    nlgpu.softmax_rows(nlgpu.to_device(a), dc, rows, n)
+    got = dc.download(np.float32, rows * n).reshape(rows, n)
+    e = np.exp(a.astype(np.float64) - a.max(axis=1, keepdims=True))
+    exact = e / e.sum(axis=1, keepdims=True)
+    assert np.max(np.abs(got - exact) / np.maximum(exact, 1e-30)) <= 1e-5
