@@ -15,6 +15,7 @@ lisp/nelisp-gpu-kernels.el:700-746) and a seeded counter-based generator
 from __future__ import annotations
 
 import ctypes as C
+import gc
 import os
 from typing import Iterable, Optional, Sequence
 
@@ -584,6 +585,7 @@ class Event:
 
 
 def graph_begin(stream=None) -> None:
+    gc.collect()  # arrays in dead cycles: a device free inside a capture would end it
     _check(lib().nlg_graph_begin(stream), "graph_begin")
 
 

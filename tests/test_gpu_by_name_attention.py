@@ -6,6 +6,8 @@ and NaNs after a query, and buffers that take the general kernel instead.
 decode-attn(-b) on its split form likewise: every lanes-per-row form, one and
 many workgroups per head (a call under capture takes one), positions at the
 edges of its blocks and past the cache, NaN in every row not attended."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -296,6 +298,27 @@ def test_decode_attention_f32_general_form():
     want = out.copy()
     orc.dispatch("decode-attn-b", [q.copy(), k[:k.size - 70].copy(), v.copy(), np.array([pos], f32), want], push, 4)
     assert np.max(np.abs(devs[-1].download(f32, out.size) - want)) <= 1e-5 * np.max(np.abs(want))
+
+
+def test_a_collection_inside_a_capture_frees_nothing():
+    """An array that only a dead reference cycle holds is freed before a capture
+    begins, not by a collection that falls inside it."""
+    x = np.arange(256, dtype=f32)
+    devs = [nlgpu.to_device(b) for b in (x, x, np.zeros(256, f32))]
+    s = nlgpu.lib().nlg_stream_create()
+    cycle = [nlgpu.DeviceArray(4096)]
+    cycle.append(cycle)
+    del cycle
+    nlgpu.graph_begin(s)
+    gc.collect()
+    nlgpu.dispatch("vadd", devs, [256], 4, stream=s)
+    g = nlgpu.graph_end(s)
+    for _ in range(3):
+        nlgpu.graph_launch(g, s)
+        nlgpu.sync(s)
+        assert np.array_equal(devs[2].download(f32, 256), 2 * x)
+    nlgpu.graph_destroy(g)
+    nlgpu.lib().nlg_stream_destroy(s)
 
 
 def test_decode_attention_f32_beside_a_capture():
