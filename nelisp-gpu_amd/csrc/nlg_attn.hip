@@ -365,7 +365,9 @@ static bool decode_split(const DecArgs &a, hipStream_t st) {
   sa.hgroups = (a.grp + g - 1) / g;
   sa.nsplit = 1;
   // two workgroups per CU, none with less than a block for each wave
-  const uint64_t units = (uint64_t)a.B * a.kvheads * sa.hgroups, rows = a.maxseq ? a.maxseq : a.ck.n / a.kvdim;
+  const uint64_t units = (uint64_t)a.B * a.kvheads * sa.hgroups;
+  if (!nlg_fits(units, 64 * DS_WAVES)) return false;  // (k_decode_attn's workgroups are half as large)
+  const uint64_t rows = a.maxseq ? a.maxseq : a.ck.n / a.kvdim;
   const uint32_t pb = DS_NI * (a.hd <= 64 ? 4u : a.hd <= 128 ? 2u : 1u);
   uint64_t want = 2ull * nlg_num_cu() / units, most = (rows + DS_WAVES * pb - 1) / (DS_WAVES * pb);
   if (want > DS_MAX_SPLIT) want = DS_MAX_SPLIT;
@@ -707,7 +709,8 @@ __global__ __launch_bounds__(64 * GQA_NW) void k_gqa_mfma(GqaArgs a) {
 static bool gqa_mfma_ok(const GqaArgs &a) {
   const uint64_t rows = (uint64_t)a.heads * a.seq, qn = rows * a.hd, kn = (uint64_t)a.seq * a.kvheads * a.hd;
   const uintptr_t at = (uintptr_t)a.q.p | (uintptr_t)a.k.p | (uintptr_t)a.ctx;
-  return a.heads && a.heads % a.kvheads == 0 && rows < (1u << 31) && a.q.n >= qn && a.nctx >= qn &&
+  return a.heads && a.heads % a.kvheads == 0 && rows < (1u << 31) &&
+         nlg_fits(((uint64_t)a.seq + 31) / 32 * a.heads, 64 * GQA_NW) && a.q.n >= qn && a.nctx >= qn &&
          a.k.n >= kn && a.v.n >= kn && a.q.p && a.k.p && a.v.p && a.ctx && (at & 15) == 0;
 }
 

@@ -54,6 +54,9 @@ static inline uint32_t nlg_blocks(uint64_t n, uint64_t per) {
   return (uint32_t)b;
 }
 
+// Whether a grid's x dimension holds `blocks` workgroups (fewer than 2^32 threads).
+static inline bool nlg_fits(uint64_t blocks, uint32_t threads) { return blocks * threads < (1ull << 32); }
+
 // ---------------------------------------------------------------- device side
 
 // (uint f) of the DSL: OpConvertFToS into a uint (lisp/nelisp-gpu-compile.el:327).

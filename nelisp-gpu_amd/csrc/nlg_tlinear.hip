@@ -353,7 +353,7 @@ bool rows_t_mfma(const TArgs &a, hipStream_t st) {
   // is shorter (21 us a round of workgroups against 51 at 2,560 rows and any
   // position count up to 32)
   const uint64_t chains = (uint64_t)((a.cols + 63) / 64) * a.seq;
-  if (chains <= 2u * nlg_num_cu()) return false;
+  if (chains <= 2u * nlg_num_cu() || !nlg_fits((uint64_t)((a.cols + 31) / 32) * ((a.seq + 31) / 32), 256)) return false;
   // 16 columns a wave once there is one for three SIMDs of four: 6,912 columns at
   // 64 / 128 / 256 positions (432 / 864 / 1,728 such waves, the last over 6,912
   // rows) 79 / 81 / 336 us against 55 / 83 / 392 with 8 columns

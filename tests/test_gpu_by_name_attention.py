@@ -228,6 +228,20 @@ def test_decode_attention_f32_partial_grid_and_single():
     assert np.max(np.abs(devs[-1].download(f32, out.size) - want)) <= 1e-5 * np.max(np.abs(want))
 
 
+def test_decode_attention_f32_more_units_than_a_grid_holds():
+    """2^23 (sequence, kv head) pairs: 512 threads each are more than a grid's x
+    dimension holds, 256 are not."""
+    batch, heads, hd = 1 << 21, 4, 4
+    n = batch * heads * hd
+    print(f"[gpu] decode-attn-b batch={batch}", flush=True)
+    v = np.random.default_rng(3).standard_normal(n).astype(f32)
+    dv = nlgpu.to_device(v)
+    out = nlgpu.to_device(np.zeros(n, f32))
+    nlgpu.dispatch("decode-attn-b", [dv, dv, dv, nlgpu.to_device(np.array([0], f32)), out], [batch, heads * hd, heads, heads, 1],
+                   n // 64)
+    assert np.array_equal(out.download(f32, n), v)  # one position: its values
+
+
 def test_decode_attention_f32_infinities():
     """An attended V of infinities and an attended K whose score is NaN."""
     batch, heads, kvh, hd, maxseq, pos = 1, 4, 2, 64, 200, 150
