@@ -364,7 +364,8 @@ static bool decode_split(const DecArgs &a, hipStream_t st) {
   const uint32_t g = a.grp >= 3 ? 4u : a.grp;
   sa.hgroups = (a.grp + g - 1) / g;
   sa.nsplit = 1;
-  // two workgroups per CU, none with less than a block for each wave
+  // two workgroups per CU (for two and four heads of up to 128 the registers hold one at a
+  // time: two rounds), none with less than a block for each wave of the cache's room
   const uint64_t units = (uint64_t)a.B * a.kvheads * sa.hgroups;
   if (!nlg_fits(units, 64 * DS_WAVES)) return false;  // (k_decode_attn's workgroups are half as large)
   const uint64_t rows = a.maxseq ? a.maxseq : a.ck.n / a.kvdim;

@@ -4,7 +4,8 @@
 // caches (decode-attn(-b), kernels.el:315-338, :366-390: scale 1/sqrt(hd),
 // max seeded at -1e30, C = sum(e*V)/sum(e)), split over chunks of positions.
 // Each workgroup of the first pass handles one (chunk, kv head, sequence)
-// for all the query heads of that kv head, so K and V are read from HBM once;
+// for all the query heads of that kv head (four of eight, the other four beside
+// it on one XCD), so K and V are read from HBM once;
 // a second launch merges the chunks (max-rescaled sums).  The same chunk pass
 // serves contiguous caches [seq][kvheads][max_seq][hd], paged pools
 // (decode-attn-paged-v, kernels.el:1222-1246) through a block table, and
