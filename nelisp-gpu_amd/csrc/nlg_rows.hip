@@ -16,6 +16,24 @@
 
 #define EPS6 0.000001f
 
+// Sum over the 16 waves of a workgroup, in every thread.  The waves' sums meet in
+// pairs: added one after another, each of 15 sums as large as the result is rounded, and
+// rows whose weight lies in a few waves (causal ones) show it.
+__device__ __forceinline__ float block_sum16(float v, float *red) {
+  v = nlg_wave_sum_f32(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  float t[16];
+#pragma unroll
+  for (int i = 0; i < 16; i++) t[i] = red[i];
+#pragma unroll
+  for (int n = 8; n; n /= 2)
+#pragma unroll
+    for (int i = 0; i < n; i++) t[i] = t[2 * i] + t[2 * i + 1];
+  return t[0];
+}
+
 // The reference's max starts from the first element and only moves on a
 // strict `>`: NaNs are never selected, except that a NaN first element stays.
 // TPR threads take a row and hold EPT of its values each: a wave (no LDS, no
@@ -25,6 +43,7 @@ __global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void k_softmax_reg(const flo
                                                                       uint32_t n) {
   __shared__ float red[TPR < 256 ? 1 : TPR / 64];
   constexpr bool WAVE = TPR == 64;
+  constexpr bool PAIRS = WAVE && V4 && EPT == 16;  // a lane's chain as long as with four times the lanes
   const uint32_t tid = threadIdx.x % TPR;
   const uint32_t row = WAVE ? blockIdx.x * 4 + threadIdx.x / 64 : blockIdx.x;
   if (row >= rows) return;
@@ -57,9 +76,13 @@ __global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void k_softmax_reg(const flo
   for (int k = 0; k < EPT; k++) {
     const uint32_t i = V4 ? 4 * (tid + TPR * (k / 4)) + (k % 4) : tid + TPR * k;
     v[k] = expf(__fsub_rn(v[k], mx));
-    if (i < n) s = __fadd_rn(s, v[k]);
+    if (PAIRS) {
+      if (k % 4 == 3 && i < n) s += (v[k - 3] + v[k - 2]) + (v[k - 1] + v[k]);
+    } else if (i < n) {
+      s = __fadd_rn(s, v[k]);
+    }
   }
-  s = WAVE ? nlg_wave_sum_f32(s) : nlg_block_sum_f32(s, red);
+  s = WAVE ? nlg_wave_sum_f32(s) : TPR == 1024 ? block_sum16(s, red) : nlg_block_sum_f32(s, red);
   if (V4) {
 #pragma unroll
     for (int k = 0; k < EPT / 4; k++) {
